@@ -1,0 +1,450 @@
+// bfa_panel.hip -- register-resident LU panel: an m x w block column (w up to
+// 256) factored with partial pivoting by one launch of co-resident
+// workgroups, one exchange through memory per column.
+//
+// Replaces the column loop of HMatrix::LUFactorize's zgetrf
+// (src/applications/buff-scatter/buff-scatter.cc:285).
+#include <hip/hip_runtime.h>
+#include <algorithm>
+
+#include "bfa_internal.h"
+#include "bfa_panel.h"
+
+using namespace bfa;
+
+namespace {
+
+template <typename T> struct zc { T re, im; };
+template <typename T> __device__ __forceinline__ zc<T> z_mul(zc<T> a, zc<T> b)
+{ return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
+template <typename T> __device__ __forceinline__ T t_fma(T a, T b, T c) { return sizeof(T) == 8 ? (T)fma(a, b, c) : (T)fmaf(a, b, c); }
+// a - l u
+template <typename T> __device__ __forceinline__ zc<T> z_fms(zc<T> a, zc<T> l, zc<T> u)
+{ return {t_fma(l.im, u.im, t_fma(-l.re, u.re, a.re)), t_fma(-l.im, u.re, t_fma(-l.re, u.im, a.im))}; }
+template <typename T> __device__ __forceinline__ zc<T> z_pick(bool c, zc<T> a, zc<T> b)
+{ return {c ? a.re : b.re, c ? a.im : b.im}; }
+template <typename T> __device__ __forceinline__ T z_abs1(zc<T> a) { return fabs(a.re) + fabs(a.im); }
+
+// agent-scope relaxed accesses: coherent between workgroups of one launch
+// wherever they run, no cache maintenance
+__device__ __forceinline__ void ag_store(unsigned long long *p, unsigned long long v)
+{ __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ unsigned long long ag_load(const unsigned long long *p)
+{ return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// a row entry travels as 8-byte words of 32 data bits below the column's
+// 32-bit sequence number, so that every word proves itself current; word k of
+// all entries together (XP_PLANE apart), so that a wave's accesses are whole
+// lines
+__device__ __forceinline__ void put_word(unsigned long long *p, unsigned d, unsigned seq)
+{ ag_store(p, ((unsigned long long)seq << 32) | d); }
+__device__ __forceinline__ void put_entry(unsigned long long *p, zc<double> v, unsigned seq)
+{
+  const unsigned long long a = (unsigned long long)__double_as_longlong(v.re),
+                           b = (unsigned long long)__double_as_longlong(v.im);
+  put_word(p, (unsigned)a, seq);
+  put_word(p + XP_PLANE, (unsigned)(a >> 32), seq);
+  put_word(p + 2 * XP_PLANE, (unsigned)b, seq);
+  put_word(p + 3 * XP_PLANE, (unsigned)(b >> 32), seq);
+}
+__device__ __forceinline__ void put_entry(unsigned long long *p, zc<float> v, unsigned seq)
+{
+  put_word(p, __float_as_uint(v.re), seq);
+  put_word(p + XP_PLANE, __float_as_uint(v.im), seq);
+}
+// false while a word is not yet the column's
+__device__ __forceinline__ bool get_entry(const unsigned long long *p, zc<double> &v, unsigned seq)
+{
+  const unsigned long long a = ag_load(p), b = ag_load(p + XP_PLANE), c = ag_load(p + 2 * XP_PLANE),
+                           d = ag_load(p + 3 * XP_PLANE);
+  v = {__longlong_as_double((long long)((a & 0xffffffffull) | (b << 32))),
+       __longlong_as_double((long long)((c & 0xffffffffull) | (d << 32)))};
+  return (unsigned)(a >> 32) == seq && (unsigned)(b >> 32) == seq && (unsigned)(c >> 32) == seq &&
+         (unsigned)(d >> 32) == seq;
+}
+__device__ __forceinline__ bool get_entry(const unsigned long long *p, zc<float> &v, unsigned seq)
+{
+  const unsigned long long a = ag_load(p), b = ag_load(p + XP_PLANE);
+  v = {__uint_as_float((unsigned)a), __uint_as_float((unsigned)b)};
+  return (unsigned)(a >> 32) == seq && (unsigned)(b >> 32) == seq;
+}
+// 1 / a: on the path from one exchange to the next, so the reciprocal of
+// |a|^2 comes from the hardware estimate and two Newton steps where that
+// cannot overflow, in place of two divisions
+__device__ __forceinline__ double recip(double d)
+{
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  return fma(y, fma(-d, y, 1.0), y);
+}
+__device__ __forceinline__ float recip(float d)
+{
+  const float y = __builtin_amdgcn_rcpf(d);
+  return fmaf(y, fmaf(-d, y, 1.0f), y);
+}
+template <typename T> __device__ __forceinline__ zc<T> z_inv(zc<T> a)
+{
+  constexpr T big = sizeof(T) == 8 ? (T)1e290 : (T)1e30;
+  const T d = a.re * a.re + a.im * a.im;
+  if (d > 1 / big && d < big) {
+    const T y = recip(d);
+    return {a.re * y, -a.im * y};
+  }
+  return {a.re / d, -a.im / d};
+}
+
+// value of lane `src` (wave-uniform)
+__device__ __forceinline__ float lane_get(float v, int src)
+{ return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), src)); }
+__device__ __forceinline__ double lane_get(double v, int src)
+{
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, src), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), src);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <typename T> __device__ __forceinline__ zc<T> lane_get(zc<T> v, int src)
+{ return {lane_get(v.re, src), lane_get(v.im, src)}; }
+
+template <int CTRL> __device__ __forceinline__ unsigned dpp_max(unsigned v)
+{
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+  return o > v ? o : v;
+}
+// maximum over the wave: row shifts, then the two row broadcasts
+__device__ __forceinline__ unsigned wave_max(unsigned v)
+{
+  v = dpp_max<0x111>(v);
+  v = dpp_max<0x112>(v);
+  v = dpp_max<0x114>(v);
+  v = dpp_max<0x118>(v);
+  v = dpp_max<0x142>(v);
+  v = dpp_max<0x143>(v);
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// a[i] for a wave-uniform i: a branch tree down to four rows, then selects (an
+// array indexed by a variable would be moved to scratch memory; the leaves'
+// distinct comments keep them from being merged into such an access)
+template <int LO, int HI, typename T, int R> __device__ __forceinline__ void reg_get(const zc<T> (&a)[R], int i, zc<T> &x)
+{
+  if constexpr (HI - LO <= 4) {
+    x = a[LO];
+#pragma unroll
+    for (int k = LO + 1; k < HI; k++) x = z_pick(i == k, a[k], x);
+    asm volatile("; leaf %2" : "+v"(x.re), "+v"(x.im) : "i"(LO));
+  } else {
+    constexpr int MID = LO + ((HI - LO) / 4 + 1) / 2 * 4;
+    if (i < MID) reg_get<LO, MID>(a, i, x);
+    else reg_get<MID, HI>(a, i, x);
+  }
+}
+template <int LO, int HI, typename T, int R> __device__ __forceinline__ void reg_put(zc<T> (&a)[R], int i, zc<T> x)
+{
+  if constexpr (HI - LO <= 4) {
+#pragma unroll
+    for (int k = LO; k < HI; k++) a[k] = z_pick(i == k, x, a[k]);
+    asm volatile("; leaf %0" : : "i"(LO));
+  } else {
+    constexpr int MID = LO + ((HI - LO) / 4 + 1) / 2 * 4;
+    if (i < MID) reg_put<LO, MID>(a, i, x);
+    else reg_put<MID, HI>(a, i, x);
+  }
+}
+
+#define XP_NT 256
+#define XP_SPIN_LIMIT (1u << 22)
+
+template <typename T, int NR> struct XpShared { zc<T> col[4][NR]; };
+
+// One workgroup (rank of nwg) of the panel.  Thread (h, t) holds rows
+// r0 + h R .. r0 + h R + R - 1 of column t in registers for the whole panel;
+// lanes also hold, redundantly in every wave, the next two columns row by row
+// (lane = row), so that the multipliers of column j, the values of column
+// j + 1 and its pivot candidate need no workgroup reduction.
+//
+// Exchange of column j: the owner of row j publishes that row (all columns) as
+// soon as it is up to date; every workgroup publishes one word {sequence
+// number, magnitude, row} of its candidate and, behind it, the candidate's
+// row.  Every wave reads all workgroups' words until they carry this column's
+// sequence number, so all see the same pivot (largest |re| + |im| rounded to
+// float, first row among equals, as izamax does), and row j with them; only a
+// pivot elsewhere costs a further read.  A row's words carry the sequence
+// number as well: no store is waited for and nothing is cleared, the numbers
+// never repeat between launches.  The register update of column j - 1
+// overlaps the exchange.
+// Words and rows rotate through XP_NBUF buffers: wave 0 publishes column
+// j + 2 after the workgroup barrier of column j, which every wave passes only
+// when it has read column j's, so a workgroup that has seen all words of
+// j + 2 may overwrite column j's.
+//
+// Rows that are finished (global row <= j) are left out of the update.  The
+// multipliers of column j go to A straight from the lanes, in the row order of
+// step j: the interchanges of later columns are applied to them afterwards,
+// with those of the columns left of the panel (k_laswp_left); U is written at
+// the end.
+template <typename T, int WB, int R>
+__device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<T, (XP_NT / WB) * R> &sh)
+{
+  constexpr int NH = XP_NT / WB, NR = NH * R, EW = sizeof(T) / 2;   // EW: words of an entry
+  typedef zc<T> Z;
+  typedef unsigned long long u64;
+  __builtin_amdgcn_s_setprio(3);
+  const int tid = threadIdx.x, lane = tid & 63, t = tid % WB;
+  const int h = __builtin_amdgcn_readfirstlane(tid / WB), t0 = __builtin_amdgcn_readfirstlane(t & ~63);
+  const int m = p.m, w = p.w, nwg = p.nwg, r0 = rank * NR;
+  Z *A = (Z *)p.A;
+  Z a[R];
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    const int r = r0 + h * R + i;
+    a[i] = (t < w && r < m) ? A[(size_t)t * p.lda + r] : Z{0, 0};
+  }
+  // columns 0, 1 to the lanes; column 2 waits in buffer 0
+  if (t < 3) {
+#pragma unroll
+    for (int i = 0; i < R; i++) sh.col[t][h * R + i] = a[i];
+  }
+  __syncthreads();
+  Z c0[NH], c1[NH], l[NH];
+#pragma unroll
+  for (int q = 0; q < NH; q++) {
+    const int i = q * R + (lane < R ? lane : 0);
+    c0[q] = sh.col[0][i];
+    c1[q] = sh.col[1][i];
+    l[q] = {0, 0};
+  }
+  Z pt = {0, 0};
+  bool dead = false;               // a wait gave up somewhere: finish without waiting
+  auto wait_ok = [&](unsigned &spins) __attribute__((always_inline)) {
+    if (dead) return true;
+    if ((++spins & 255) == 0 && __hip_atomic_load(&p.err[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) dead = true;
+    if (spins > XP_SPIN_LIMIT) {
+      if (lane == 0) atomicOr(&p.err[0], 1);   // reported as an error by the host
+      dead = true;
+    }
+    return dead;
+  };
+  auto row_slot = [&](int buf, int who) __attribute__((always_inline)) {
+    return (u64 *)p.data + ((size_t)buf * (XP_MAXWG + 1) + who) * XP_PLANE * EW;
+  };
+  // row jn's register values before step jn - 1, fetched while waiting (the
+  // owner's wave half only)
+  Z xn = {0, 0};
+  auto fetch = [&](int jn) __attribute__((always_inline)) {
+    if (jn >= r0 && jn < r0 + NR && h == (jn - r0) / R) reg_get<0, R>(a, (jn - r0) % R, xn);
+  };
+  // row `row` of this workgroup, whose register values (x) miss step jn - 1 if elim
+  auto send = [&](int row, Z x, u64 *dst, unsigned seq, bool elim) __attribute__((always_inline)) {
+    Z lx = {0, 0};
+#pragma unroll
+    for (int q = 0; q < NH; q++)
+      if (q == h) lx = lane_get(l[q], row % R);
+    if (elim) x = z_fms(x, lx, pt);
+    put_entry(dst + t, x, seq);
+  };
+  // row jn, then the candidate of column jn (lanes hold the column in c0)
+  auto publish = [&](int jn, bool elim) __attribute__((always_inline)) {
+    const unsigned seq = p.seq0 + jn;
+    const int buf = jn & (XP_NBUF - 1), lj = jn - r0;
+    if (lj >= 0 && lj < NR && h == lj / R) send(lj, xn, row_slot(buf, XP_MAXWG), seq, elim);
+    unsigned mg[NH], mx = 0;
+#pragma unroll
+    for (int q = 0; q < NH; q++) {
+      const int r = r0 + q * R + lane;
+      const float v = (float)z_abs1(c0[q]);
+      mg[q] = (lane < R && r < m && r >= jn) ? (v == v ? __float_as_uint(v) : 0u) + 1u : 0u;
+      mx = mg[q] > mx ? mg[q] : mx;
+    }
+    const unsigned M = wave_max(mx);
+    int rp = -1;
+    if (M) {
+#pragma unroll
+      for (int q = NH - 1; q >= 0; q--) {
+        const u64 b = __ballot(mg[q] == M);
+        if (b) rp = q * R + (int)__builtin_ctzll(b);
+      }
+    }
+    if (tid == 0)
+      ag_store(p.flags + ((size_t)buf * XP_MAXWG + rank) * XP_FSTRIDE,
+               ((u64)seq << 40) | ((u64)M << 9) | (unsigned)(rp < 0 ? 0 : rp));
+    if (rp >= 0 && rp != lj && h == rp / R) {
+      Z x;
+      reg_get<0, R>(a, rp % R, x);
+      send(rp, x, row_slot(buf, rank), seq, elim);
+    }
+  };
+  fetch(0);
+  publish(0, false);
+  fetch(1);
+#pragma unroll 1
+  for (int j = 0; j < w; j++) {
+    const int buf = j & (XP_NBUF - 1);
+    const unsigned seq = p.seq0 + j;
+    // every workgroup's candidate; beside it row j, which most often is the
+    // pivot's (and otherwise moves to the pivot's place): this thread's column,
+    // and columns j, j + 1, j + 2 once more on lanes 0 .. 2
+    const int ib = min(j + (lane & 3), WB - 1);
+    const u64 *fl = p.flags + (size_t)buf * XP_MAXWG * XP_FSTRIDE, *rj = row_slot(buf, XP_MAXWG);
+    const bool two = nwg > 64;
+    u64 f, f2 = 0;
+    Z rt, rb;
+    bool have = false;
+    for (unsigned spins = 0;;) {
+      f = lane < nwg ? ag_load(fl + (size_t)lane * XP_FSTRIDE) : (u64)seq << 40;
+      if (two) f2 = lane + 64 < nwg ? ag_load(fl + (size_t)(lane + 64) * XP_FSTRIDE) : (u64)seq << 40;
+      if (!have) {
+        const bool a1 = get_entry(rj + t, rt, seq), a2 = get_entry(rj + ib, rb, seq);
+        have = __ballot(a1 && a2) == ~0ull;
+      }
+      const bool all = __ballot((unsigned)(f >> 40) == seq && (!two || (unsigned)(f2 >> 40) == seq)) == ~0ull;
+      if ((all && have) || wait_ok(spins)) break;
+    }
+    const unsigned mg = lane < nwg ? (unsigned)(f >> 9) & 0x7fffffffu : 0u;
+    const unsigned mg2 = two && lane + 64 < nwg ? (unsigned)(f2 >> 9) & 0x7fffffffu : 0u;
+    const unsigned M = wave_max(mg > mg2 ? mg : mg2);
+    const u64 wb = __ballot(lane < nwg && mg == M), wb2 = __ballot(mg2 == M);
+    int win, lrow;
+    if (wb) {
+      win = (int)__builtin_ctzll(wb);
+      lrow = (int)(__builtin_amdgcn_readlane((unsigned)f, win) & 511u);
+    } else {
+      win = wb2 ? (int)__builtin_ctzll(wb2) : 0;
+      lrow = (int)(__builtin_amdgcn_readlane((unsigned)f2, win) & 511u);
+      win = min(win + 64, nwg - 1);
+    }
+    const int prow = max(j, min(m - 1, win * NR + lrow));
+    const bool ownp = prow != j && prow >= r0 && prow < r0 + NR;
+    Z pb = rb;
+    pt = rt;
+    if (prow != j) {
+      const u64 *pr = row_slot(buf, win);
+      for (unsigned spins = 0;;) {
+        const bool a1 = get_entry(pr + t, pt, seq), a2 = get_entry(pr + ib, pb, seq);
+        if (__ballot(a1 && a2) == ~0ull || wait_ok(spins)) break;
+      }
+    }
+    const Z pj = lane_get(pb, 0), pj1 = lane_get(pb, 1), pj2 = lane_get(pb, 2), inv = z_inv(pj);
+    // rows j and prow change places
+    const int lp = prow - r0;
+    if (prow != j) {
+      const int lj = j - r0;
+      if (lj >= 0 && lj < NR && h == lj / R) reg_put<0, R>(a, lj % R, pt);
+      if (ownp) {
+        if (h == lp / R) reg_put<0, R>(a, lp % R, rt);
+        if (lp == j + 1 - r0) xn = rt;
+        const Z r0v = lane_get(rb, 0), r1v = lane_get(rb, 1);
+#pragma unroll
+        for (int q = 0; q < NH; q++)
+          if (q * R + lane == lp && lane < R) { c0[q] = r0v; c1[q] = r1v; }
+      }
+    }
+    if (t <= j) pt = {0, 0};       // finished columns: the update below leaves them alone
+    const bool scale = z_abs1(pj) != (T)0;
+    Z lo[NH];                       // column j of L as stored
+#pragma unroll
+    for (int q = 0; q < NH; q++) {
+      const bool act = lane < R && r0 + q * R + lane > j;
+      l[q] = scale && act ? z_mul(c0[q], inv) : Z{0, 0};
+      lo[q] = z_pick(scale, l[q], c0[q]);
+      c0[q] = scale && act ? z_fms(c1[q], l[q], pj1) : c1[q];
+    }
+    if (j + 1 < w) publish(j + 1, scale);
+    if ((tid >> 6) == (j & (XP_NT / 64 - 1))) {
+#pragma unroll
+      for (int q = 0; q < NH; q++) {
+        const int r = r0 + q * R + lane;
+        if (lane < R && r > j && r < m) A[(size_t)j * p.lda + r] = lo[q];
+      }
+    }
+    if (rank == 0 && tid == 0) {
+      p.ipiv[j] = prow + p.piv_off;
+      if (!scale && p.err[1] == 0) p.err[1] = p.piv_off + j + 1;
+    }
+    __syncthreads();
+    // column j + 2 (through step j - 1) from its buffer, then step j
+#pragma unroll
+    for (int q = 0; q < NH; q++) {
+      const int i = q * R + (lane < R ? lane : 0);
+      Z v = sh.col[2 + (j & 1)][i];
+      if (ownp && i == lp) v = lane_get(rb, 2);
+      const bool act = lane < R && r0 + i > j;
+      c1[q] = scale && act ? z_fms(v, l[q], pj2) : v;
+    }
+    // the other rows
+    const int ist = max(0, j + 1 - r0 - h * R);
+    if (scale && ist < R && t0 + 63 > j) {
+      Z ls = l[0];
+#pragma unroll
+      for (int q = 1; q < NH; q++)
+        if (q == h) ls = l[q];
+      if (ist == 0) {
+#pragma unroll
+        for (int i = 0; i < R; i++) a[i] = z_fms(a[i], lane_get(ls, i), pt);
+      } else {
+#pragma unroll
+        for (int i = 1; i < R; i++) a[i] = z_pick(i >= ist, z_fms(a[i], lane_get(ls, i), pt), a[i]);
+      }
+    }
+    if (t == j + 3) {
+#pragma unroll
+      for (int i = 0; i < R; i++) sh.col[2 + ((j + 1) & 1)][h * R + i] = a[i];
+    }
+    fetch(j + 2);
+  }
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    const int r = r0 + h * R + i;
+    if (t < w && r <= t && r < m) A[(size_t)t * p.lda + r] = a[i];
+  }
+}
+
+template <typename T, int WB, int R> __global__ __launch_bounds__(XP_NT) void k_xpanel(XPanel p)
+{
+  __shared__ XpShared<T, (XP_NT / WB) * R> sh;
+  xpanel_body<T, WB, R>(p, blockIdx.x, sh);
+}
+
+template <typename T, int WB, int R> void launch(XPanel p, hipStream_t st)
+{
+  p.nwg = (p.m + XP_NT / WB * R - 1) / (XP_NT / WB * R);
+  hipLaunchKernelGGL((k_xpanel<T, WB, R>), dim3(p.nwg), dim3(XP_NT), 0, st, p);
+}
+
+}  // namespace
+
+namespace bfa {
+static const size_t kRowBytes = (size_t)XP_NBUF * (XP_MAXWG + 1) * XP_PLANE * 32;
+size_t xpanel_bytes() { return kRowBytes + (size_t)XP_NBUF * XP_MAXWG * XP_FSTRIDE * 8; }
+
+void xpanel_carve(char *mem, XPanel *p)
+{
+  p->data = mem;
+  p->flags = (unsigned long long *)(mem + kRowBytes);
+}
+
+// Rows a workgroup holds, fewest first: a column's time grows with them (the
+// register update outlasts the exchange from about 16 complex128 / 32
+// complex64 rows), the exchange's hardly with the workgroups.  Measured, us a
+// column of 256: complex128 1.76 (8 rows, m = 256), 1.99 (16, 1,350), 2.4
+// (24, 3,000), 2.6 (32, 1,350); complex64 1.53 (8, 256), 1.73 (16, 1,350),
+// 2.2 (32, 4,000), 2.6 (48, 6,000).
+int xpanel_max_rows(bool f64) { return XP_MAXWG * (f64 ? 32 : 48); }
+
+int launch_xpanel(bool f64, XPanel p, hipStream_t st)
+{
+  if (p.m < 1 || p.m > xpanel_max_rows(f64) || p.w < 1 || p.w > XP_MAXW || p.w > p.m)
+    return fail(BFA_ERR_ARG, "register panel of %d x %d", p.m, p.w);
+  if (f64) {
+    if (p.m <= XP_MAXWG * 8) launch<double, 256, 8>(p, st);
+    else if (p.m <= XP_MAXWG * 16) launch<double, 256, 16>(p, st);
+    else if (p.m <= XP_MAXWG * 24) launch<double, 256, 24>(p, st);
+    else launch<double, 256, 32>(p, st);
+  } else {
+    if (p.m <= XP_MAXWG * 8) launch<float, 256, 8>(p, st);
+    else if (p.m <= XP_MAXWG * 16) launch<float, 256, 16>(p, st);
+    else if (p.m <= XP_MAXWG * 32) launch<float, 256, 32>(p, st);
+    else launch<float, 256, 48>(p, st);
+  }
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? BFA_OK : fail(BFA_ERR_HIP, "register panel launch: %s", hipGetErrorString(e));
+}
+}  // namespace bfa

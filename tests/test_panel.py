@@ -1,0 +1,80 @@
+"""Register-resident LU panel (bfa_panel.hip) at the sizes where its workgroup
+shape changes: one row, the edges of a 256-column panel, the first size of each
+rows-a-workgroup variant, and the largest matrix that takes it whole."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+
+def _load():
+    import __graft_entry__ as ge
+    return ge._load_pkg()
+
+
+def _factor(bfa, A, f64):
+    """LU of the matrix whose column-major storage is A (A[c, r] = M(r, c))."""
+    n = len(A)
+    piv = torch.zeros(n, dtype=torch.int32, device="cuda")
+    info = (bfa.lu_factor if f64 else bfa.lu_factor_c)(A, n, piv)
+    return info, piv.cpu().numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f64", [True, False])
+@pytest.mark.parametrize("n", [1, 2, 65, 255, 257, 600, 1025, 2049, 3073, 4097])
+def test_panel_backward_error_and_pivots(n, f64):
+    bfa = _load()
+    rng = np.random.default_rng(n)
+    dt = np.complex128 if f64 else np.complex64
+    M = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))).astype(dt)
+    A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+    info, piv = _factor(bfa, A, f64)
+    assert info == 0
+    LU = A.T.to(torch.complex128)
+    L = torch.tril(LU, -1) + torch.eye(n, dtype=LU.dtype, device="cuda")
+    U = torch.triu(LU)
+    perm = np.arange(n)
+    for i, p in enumerate(piv):
+        assert i <= p < n
+        perm[[i, p]] = perm[[p, i]]
+    PA = torch.from_numpy(M[perm].astype(np.complex128)).cuda()
+    # |PA - LU| <= gamma_n |L||U| entry by entry, gamma_n = n sqrt(8) u for complex arithmetic; in norms
+    u = np.finfo(np.float64 if f64 else np.float32).eps / 2
+    bound = n * np.sqrt(8.0) * u * torch.linalg.norm(L.abs() @ U.abs())
+    assert torch.linalg.norm(PA - L @ U) <= bound
+    # partial pivoting: no multiplier is larger than its pivot in |re| + |im| (izamax's norm): |l| <= sqrt(2),
+    # and the float rounding of the compared magnitudes
+    assert L.abs().max() <= np.sqrt(2.0) * (1 + 1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [40, 300])
+def test_panel_equals_lapack_pivots_and_ties(n):
+    """The first of equal magnitudes wins, as izamax chooses it; a permuted identity needs every interchange."""
+    bfa = _load()
+    import scipy.linalg as sl
+    rng = np.random.default_rng(3)
+    P = np.eye(n)[rng.permutation(n)].astype(np.complex128)
+    S = rng.choice([1.0, -1.0, 1j, -1j], (n, n)) + 4.0 * P      # many equal magnitudes
+    for M in (P, S):
+        A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+        info, piv = _factor(bfa, A, True)
+        assert info == 0
+        ref = sl.lu_factor(M)[1]
+        same = piv == ref
+        # rounding decides ties after the first steps in S; the permutation has none
+        assert same.all() if M is P else same[0]
+
+
+@pytest.mark.gpu
+def test_panel_zero_column_reports_info():
+    bfa = _load()
+    n = 300
+    rng = np.random.default_rng(5)
+    M = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    M[:, 270] = 0.0
+    A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+    info, piv = _factor(bfa, A, True)
+    assert info == 271
+    assert bool(torch.isfinite(torch.view_as_real(A)).all())
