@@ -26,6 +26,8 @@
 #include "bfa_group.h"
 #include "bfa_rules.h"
 #include "bfa_expr.h"
+#include "bfa_math.h"
+#include "bfa_power.h"
 #define TD_QUAL __constant__
 #include "td_regions.h"
 
@@ -643,17 +645,6 @@ struct FarTpShared {
   double cen[2][3][2 * FT2];
   int slot[2][2 * FT2];          // (BF local * 2 + side) -> distinct tet
 };
-
-// 1/sqrt(x): the hardware estimate (v_rsq_f64, ~23 correct bits) refined by
-// two Newton steps y <- y + y/2 (1 - x y^2) to full double precision;
-// replaces a correctly rounded sqrt and a division in the pair loop
-__device__ __forceinline__ double rsqrt_nr(double x)
-{
-  double y = __builtin_amdgcn_rsq(x);
-  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-  return y;
-}
 
 // 4-point product-rule moments of one tetrahedron pair (signed weights):
 // row tetrahedron us of the tile (points in sh), column tetrahedron's points
@@ -2059,36 +2050,31 @@ __global__ __launch_bounds__(FT_THREADS) void k_emt_q(DevGeom g, double omega, d
   emt_tp_tile(g, omega, Q, ldq, ti, tj, sh);
 }
 
-// per (a, j): y = sum_b Q_ab J_bj ; part = Re(conj(J_aj) y) + |J_aj|^2 Q_aa ; ext = Re(conj(J) <b,E>)
-__global__ void k_emt_rows(DevGeom g, double omega, const double *Q, int64_t ldq, const cd *J, int64_t ldj,
-                           PWList pws, int npw, double *partS, double *partE)
+// extinction: per (a, j) Re(conj(J_aj) <b_a, E_j>), summed over the block's rows
+__device__ __forceinline__ void emt_ext_block(const DevGeom &g, double omega, const cd *Jj, const bfa_planewave &pw,
+                                              int blk, double *out)
 {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y;
-  __shared__ double rs[256], re[256];
-  double s = 0.0, e = 0.0;
+  __shared__ double re[256];
+  const int a = blk * 256 + threadIdx.x;
+  double e = 0.0;
   if (a < g.nbf) {
-    cd y = {0.0, 0.0};
-    const cd *Jj = J + (size_t)j * ldj;
-    for (int b = 0; b < g.nbf; b++) {
-      const double q = Q[(size_t)b * ldq + a];
-      y.re += q * Jj[b].re; y.im += q * Jj[b].im;
-    }
-    const cd ja = Jj[a];
-    s = ja.re * y.re + ja.im * y.im + (ja.re * ja.re + ja.im * ja.im) * Q[(size_t)a * ldq + a];
-    const cd qe = bf_dot_pw(g, a, pws.pw[j], omega);
+    const cd qe = bf_dot_pw(g, a, pw, omega), ja = Jj[a];
     e = ja.re * qe.re + ja.im * qe.im;
   }
-  rs[threadIdx.x] = s; re[threadIdx.x] = e;
+  re[threadIdx.x] = e;
   __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) { rs[threadIdx.x] += rs[threadIdx.x + off]; re[threadIdx.x] += re[threadIdx.x + off]; }
+  for (int off = 128; off > 0; off >>= 1) {
+    if ((int)threadIdx.x < off) re[threadIdx.x] += re[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    partS[(size_t)j * gridDim.x + blockIdx.x] = rs[0];
-    partE[(size_t)j * gridDim.x + blockIdx.x] = re[0];
-  }
+  if (threadIdx.x == 0) *out = re[0];
+}
+
+__global__ __launch_bounds__(256) void k_emt_ext(DevGeom g, double omega, const cd *J, int64_t ldj, PWList pws,
+                                                 double *part)
+{
+  const int j = blockIdx.y;
+  emt_ext_block(g, omega, J + (size_t)j * ldj, pws.pw[j], blockIdx.x, part + (size_t)j * gridDim.x + blockIdx.x);
 }
 
 // ===========================================================================
@@ -2259,28 +2245,27 @@ extern "C" int bfa_emt_power(bfa_geometry *g, double omega, const bfa_planewave 
   if (omega == 0.0) return fail(BFA_ERR_ARG, "bfa_emt_power: omega = 0");
   hipStream_t st = (hipStream_t)stream;
   const int N = g->nbf;
-  double *Q = nullptr, *parts = nullptr;
+  // scattered sums [npw], extinction partials [npw][nb], then work space
   const int nb = (N + 255) / 256;
-  HIPCHECK(hipMalloc(&Q, (size_t)N * N * 8));
-  hipError_t e = hipMalloc(&parts, (size_t)2 * nb * npw * 8);
-  if (e != hipSuccess) { hipFree(Q); return fail(BFA_ERR_OOM, "bfa_emt_power: allocation failed"); }
+  const size_t nout = (size_t)npw * (nb + 1);
+  double *d = nullptr;
+  HIPCHECK(hipMalloc(&d, (nout + bfa::emt_work_doubles(g->nt, npw)) * 8));
   PWList l;
   memset(&l, 0, sizeof l);
   for (int j = 0; j < npw; j++) l.pw[j] = pw[j];
-  bfa::emt_q_matrix(g, omega, Q, N, st);
-  hipLaunchKernelGGL(k_emt_rows, dim3(nb, npw), dim3(256), 0, st, g->dg, omega, (const double *)Q, (int64_t)N,
-                     (const cd *)d_J, ldj, l, npw, parts, parts + (size_t)nb * npw);
-  std::vector<double> h((size_t)2 * nb * npw);
+  bfa::launch_emt_scattered(g->dg, omega, d_J, ldj, npw, d + nout, d, st);
+  hipLaunchKernelGGL(k_emt_ext, dim3(nb, npw), dim3(256), 0, st, g->dg, omega, (const cd *)d_J, ldj, l, d + npw);
+  std::vector<double> h(nout);
   hipError_t e1 = hipGetLastError();
-  hipError_t e2 = hipMemcpyAsync(h.data(), parts, h.size() * 8, hipMemcpyDeviceToHost, st);
+  hipError_t e2 = hipMemcpyAsync(h.data(), d, nout * 8, hipMemcpyDeviceToHost, st);
   hipError_t e3 = hipStreamSynchronize(st);
-  hipFree(Q);
-  hipFree(parts);
+  hipFree(d);
   if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess)
     return fail(BFA_ERR_HIP, "bfa_emt_power kernels failed");
   for (int j = 0; j < npw; j++) {
-    double s = 0.0, x = 0.0;
-    for (int i = 0; i < nb; i++) { s += h[(size_t)j * nb + i]; x += h[(size_t)nb * npw + (size_t)j * nb + i]; }
+    const double s = h[j];
+    double x = 0.0;
+    for (int i = 0; i < nb; i++) x += h[(size_t)npw + (size_t)j * nb + i];
     const double pscat = ZVAC * 0.5 * s;
     const double pext = 0.5 * x;
     out[2 * j] = pext - pscat;
@@ -2294,10 +2279,10 @@ extern "C" int bfa_emt_power(bfa_geometry *g, double omega, const bfa_planewave 
 // frequency comes from device memory so that one captured graph serves a
 // whole sweep.
 // ===========================================================================
-enum { GF_FAR = 0, GF_NEAR, GF_ROW, GF_EMT, GF_TAB };
+enum { GF_FAR = 0, GF_NEAR, GF_ROW, GF_TAB };
 __device__ __forceinline__ int inst_first(const AsmInst &q, int which)
 {
-  return which == GF_FAR ? q.far0 : which == GF_NEAR ? q.near0 : which == GF_ROW ? q.row0 : which == GF_EMT ? q.emt0 : q.tab0;
+  return which == GF_FAR ? q.far0 : which == GF_NEAR ? q.near0 : which == GF_ROW ? q.row0 : q.tab0;
 }
 __device__ __forceinline__ int find_inst(const AsmInst *__restrict__ d, int n, int bid, int which)
 {
@@ -2365,68 +2350,26 @@ __global__ __launch_bounds__(256) void kg_rhs(const AsmInst *__restrict__ d, int
   ((cd *)q.B)[(size_t)j * q.ldb + a] = {-v.im * s, v.re * s};
 }
 
-__global__ __launch_bounds__(FT_THREADS) void kg_emt_q(const AsmInst *__restrict__ d, int ni, const FreqState *fs)
+__global__ __launch_bounds__(256) void kg_emt_ext(const AsmInst *__restrict__ d, int ni, const FreqState *fs,
+                                                  PWBatch pws, int npw)
 {
-  __shared__ FarTpShared sh;
-  const AsmInst &q = d[find_inst(d, ni, blockIdx.x, GF_EMT)];
-  int ti, tj;
-  tile_coords(blockIdx.x - q.emt0, q.ntiles, ti, tj);
-  emt_tp_tile(q.g, fs->omega_re, q.Q, q.g.nbf, ti, tj, sh);
-}
-
-__global__ __launch_bounds__(256) void kg_emt_near(const AsmInst *__restrict__ d, int ni, const FreqState *fs)
-{
-  const AsmInst &q = d[find_inst(d, ni, blockIdx.x, GF_NEAR)];
-  const int64_t j = (int64_t)(blockIdx.x - q.near0) * blockDim.x + threadIdx.x;
-  if (j < q.g.nnz) emt_near_pair(q.g, fs->omega_re, q.Q, q.g.nbf, j);
-}
-
-__global__ __launch_bounds__(256) void kg_emt_rows(const AsmInst *__restrict__ d, int ni, const FreqState *fs,
-                                                   PWBatch pws, int npw)
-{
-  __shared__ double rs[256], re[256];
   const AsmInst &q = d[find_inst(d, ni, blockIdx.x, GF_ROW)];
   const int rb = blockIdx.x - q.row0, j = blockIdx.y;
-  const int a = rb * blockDim.x + threadIdx.x;
-  const int N = q.g.nbf;
-  const double omega = fs->omega_re;
-  double s = 0.0, e = 0.0;
-  if (a < N && j < npw) {
-    const cd *Jj = (const cd *)q.B + (size_t)j * q.ldb;
-    cd y = {0.0, 0.0};
-    for (int b = 0; b < N; b++) {
-      const double qq = q.Q[(size_t)b * N + a];
-      y.re += qq * Jj[b].re; y.im += qq * Jj[b].im;
-    }
-    const cd ja = Jj[a];
-    s = ja.re * y.re + ja.im * y.im + (ja.re * ja.re + ja.im * ja.im) * q.Q[(size_t)a * N + a];
-    const cd qe = bf_dot_pw(q.g, a, pws.pw[j], omega);
-    e = ja.re * qe.re + ja.im * qe.im;
-  }
-  rs[threadIdx.x] = s; re[threadIdx.x] = e;
-  __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) { rs[threadIdx.x] += rs[threadIdx.x + off]; re[threadIdx.x] += re[threadIdx.x + off]; }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && j < npw) {
-    q.part[(size_t)j * q.nrowblk + rb] = rs[0];
-    q.part[(size_t)(npw + j) * q.nrowblk + rb] = re[0];
-  }
+  emt_ext_block(q.g, fs->omega_re, (const cd *)q.B + (size_t)j * q.ldb, pws.pw[j], rb,
+                q.part + (size_t)(npw + j) * q.nrowblk + rb);
 }
 
-// one workgroup per instance: fixed-order sums of the row-block partials
+// one workgroup per instance: the scattered sum (part[j][0]) and the fixed-order
+// sum of the extinction's row-block partials
 __global__ __launch_bounds__(64) void kg_emt_final(const AsmInst *__restrict__ d, int ni, const FreqState *fs, int npw,
                                                    double *out)
 {
   const AsmInst &q = d[blockIdx.x];
   const int j = threadIdx.x;
   if (j >= npw) return;
-  double s = 0.0, x = 0.0;
-  for (int b = 0; b < q.nrowblk; b++) {
-    s += q.part[(size_t)j * q.nrowblk + b];
-    x += q.part[(size_t)(npw + j) * q.nrowblk + b];
-  }
+  const double s = q.part[(size_t)j * q.nrowblk];
+  double x = 0.0;
+  for (int b = 0; b < q.nrowblk; b++) x += q.part[(size_t)(npw + j) * q.nrowblk + b];
   const double pscat = ZVAC * 0.5 * s, pext = 0.5 * x;
   double *o = out + 2 * (((size_t)fs->fidx * ni + blockIdx.x) * npw + j);
   o[0] = pext - pscat;
@@ -2464,18 +2407,10 @@ void launch_rhs_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, const
 {
   if (nblk > 0) hipLaunchKernelGGL(kg_rhs, dim3(nblk, npw), dim3(256), 0, st, d, ni, fs, pw, npw);
 }
-void launch_emt_q_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, hipStream_t st)
+void launch_emt_ext_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, const PWBatch &pw, int npw,
+                      hipStream_t st)
 {
-  if (nblk > 0) hipLaunchKernelGGL(kg_emt_q, dim3(nblk), dim3(FT_THREADS), 0, st, d, ni, fs);
-}
-void launch_emt_near_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, hipStream_t st)
-{
-  if (nblk > 0) hipLaunchKernelGGL(kg_emt_near, dim3(nblk), dim3(256), 0, st, d, ni, fs);
-}
-void launch_emt_rows_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, const PWBatch &pw, int npw,
-                       hipStream_t st)
-{
-  if (nblk > 0) hipLaunchKernelGGL(kg_emt_rows, dim3(nblk, npw), dim3(256), 0, st, d, ni, fs, pw, npw);
+  if (nblk > 0) hipLaunchKernelGGL(kg_emt_ext, dim3(nblk, npw), dim3(256), 0, st, d, ni, fs, pw, npw);
 }
 void launch_emt_final_g(const AsmInst *d, int ni, const FreqState *fs, int npw, double *out, hipStream_t st)
 {

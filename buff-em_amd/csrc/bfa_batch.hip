@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "bfa_group.h"
+#include "bfa_power.h"
 #include "bfa_internal.h"
 
 using namespace bfa;
@@ -301,7 +302,7 @@ struct bfa_batch {
   int tp_state = 0;              // 0 not tried, 1 tables, -1 single pass
   // everything else in one allocation; per-instance byte offsets
   void *small = nullptr;
-  struct Off { size_t ipiv, perm, B, X, R, D, Y, Xs, inv, tick, P, norms, part, sdata, sj; };
+  struct Off { size_t ipiv, perm, B, X, R, D, Y, Xs, inv, tick, P, norms, part, emt, sdata, sj; };
   std::vector<Off> off;
   size_t o_fs = 0, o_conv = 0, o_iters = 0, o_resid = 0, o_counters = 0, o_flags = 0;
   size_t o_hist_it = 0, o_hist_res = 0, o_hist_info = 0;
@@ -843,7 +844,7 @@ std::vector<AsmInst> asm_descs(const bfa_batch *B, bool solution, int &nfar, int
     q.ldm = B->Np[i];
     q.B = solution ? (void *)B->Xp(i) : (void *)B->Bp(i);
     q.ldb = B->Np[i];
-    q.Q = (double *)B->LU32[i];   // the complex64 LU is dead once the solve is done
+    q.Q = B->at<double>(B->off[i].emt);
     q.part = B->at<double>(B->off[i].part);
     const int N = B->N[i];
     q.ntiles = (N + FT2 - 1) / FT2;
@@ -855,7 +856,7 @@ std::vector<AsmInst> asm_descs(const bfa_batch *B, bool solution, int &nfar, int
     q.nrowblk = (N + 255) / 256;
     nrow += q.nrowblk;
     q.emt0 = nemt;
-    nemt += q.ntiles * (q.ntiles + 1) / 2;
+    nemt += emt_tiles(q.g.nt);
     q.tpt = B->tp_state == 1 ? (double *)B->TP[i] : nullptr;
     q.ntb = (g->nt + 31) / 32;
     q.tab0 = ntab;
@@ -940,11 +941,10 @@ int build_plan(bfa_batch *B, double tol, int maxit)
   }
   // --- power (the complex64 LU storage becomes the EMT scratch)
   P.phase = 3;
-  P.op([B, o_emt, ni, nemt, nnear2, nrow, fs, pws, npw](hipStream_t st) {
+  P.op([B, o_emt, ni, nemt, nrow, fs, pws, npw](hipStream_t st) {
     const AsmInst *d = dp<AsmInst>(B, o_emt);
-    launch_emt_q_g(d, ni, nemt, fs, st);
-    launch_emt_near_g(d, ni, nnear2, fs, st);
-    launch_emt_rows_g(d, ni, nrow, fs, pws, npw, st);
+    launch_emt_scattered_g(d, ni, nemt, fs, npw, st);
+    launch_emt_ext_g(d, ni, nrow, fs, pws, npw, st);
     launch_emt_final_g(d, ni, fs, npw, B->power, st);
   });
   // upload descriptors
@@ -1022,6 +1022,7 @@ extern "C" int bfa_batch_create(int count, bfa_geometry *const *geoms, const bfa
     f.P = take((size_t)nchunk * npw * N * 16);
     f.norms = take((size_t)npw * nblk * 16);
     f.part = take((size_t)2 * npw * nblk * 8);
+    f.emt = take(emt_work_doubles(geoms[i]->nt, npw) * 8);
     f.sdata = take((size_t)2 * 256 * PWID * 16);
     f.sj = take(2 * PWID * 16);
     B->off.push_back(f);

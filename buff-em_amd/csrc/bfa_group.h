@@ -105,12 +105,12 @@ struct AsmInst {
   const double *table;   // static records [nnz][6]
   void *M;               // complex128 VIE matrix, N x N used, ld = ldm
   void *B;               // complex128 right-hand sides / solutions, ld = ldb
-  double *Q;             // EMT scratch, N x N doubles, ld = N
-  double *part;          // EMT partial sums [2][npw][row blocks]
+  double *Q;             // EMT work space (emt_work_doubles)
+  double *part;          // EMT sums: [0][npw][0] scattered, [1][npw][row blocks] extinction
   int64_t ldm, ldb;
   int far0, ntiles;      // far-field tiles (upper triangle of FT2 x FT2 BF tiles) from far0
   int near0, row0;       // touching-pair blocks (256) / row blocks (256)
-  int emt0, nrowblk;     // EMT Q blocks (256 entries of N x N) from emt0
+  int emt0, nrowblk;     // EMT tiles (emt_tiles) from emt0; row blocks (256)
   double *tpt;           // two-pass far field: the instance's tetrahedron-pair moment table (null: single pass)
   int tab0, ntb;         // its 32 x 32 tetrahedron tiles (upper triangle of ntb x ntb) from tab0
 };
@@ -138,10 +138,10 @@ size_t tp_table_bytes(int nt);
 void launch_near_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, bool expr, hipStream_t st);
 void launch_rhs_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, const PWBatch &pw, int npw,
                   hipStream_t st);
-void launch_emt_q_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, hipStream_t st);
-void launch_emt_near_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, hipStream_t st);
-void launch_emt_rows_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, const PWBatch &pw, int npw,
-                       hipStream_t st);
+// EMT power: the scattered sums (part[j][0]), then the extinction's row blocks
+void launch_emt_scattered_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, int npw, hipStream_t st);
+void launch_emt_ext_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, const PWBatch &pw, int npw,
+                      hipStream_t st);
 // out[(fidx * ni + i) * npw + j][2] = {P_abs, P_scat}
 void launch_emt_final_g(const AsmInst *d, int ni, const FreqState *fs, int npw, double *out, hipStream_t st);
 
