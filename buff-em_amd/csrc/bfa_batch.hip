@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "bfa_group.h"
+#include "bfa_panel.h"
 #include "bfa_power.h"
 #include "bfa_internal.h"
 
@@ -305,6 +306,7 @@ struct bfa_batch {
   struct Off { size_t ipiv, perm, B, X, R, D, Y, Xs, inv, tick, P, norms, part, emt, sdata, sj; };
   std::vector<Off> off;
   size_t o_fs = 0, o_conv = 0, o_iters = 0, o_resid = 0, o_counters = 0, o_flags = 0;
+  size_t o_xp = 0;               // register panels' exchange memory, xpanel_bytes(false) an instance
   size_t o_hist_it = 0, o_hist_res = 0, o_hist_info = 0;
   size_t ncounters = 0, ncounters_max = 0;
   double *power = nullptr;       // [nfreq][count][npw][2], grown on demand
@@ -639,6 +641,45 @@ struct Planner {
     return BFA_OK;
   }
 
+  // 256-column panels of up to xpanel_max_rows rows: register panels, as many
+  // to a launch as may run at once
+  int panel_regs(const std::vector<Pan> &ps)
+  {
+    int mmax = 0;
+    int64_t total = 0;
+    for (const Pan &p : ps) {
+      mmax = std::max(mmax, p.m);
+      total += p.m;
+    }
+    int resident = 0;
+    const int rows = xpanel_group_rows(mmax, total, &resident);
+    if (!rows) return fail(BFA_ERR_HIP, "batch: register panel occupancy query failed");
+    std::vector<XPanelProb> chunk;
+    int used = 0;
+    auto flush = [&]() {
+      if (chunk.empty()) return;
+      const size_t off = ar.put(chunk);
+      const int np = (int)chunk.size(), nblk = used;
+      op([Bp = B, off, np, nblk, rows](hipStream_t st) { launch_xpanel_g(dp<XPanelProb>(Bp, off), np, nblk, rows, st); });
+      chunk.clear();
+      used = 0;
+    };
+    for (const Pan &p : ps) {
+      const int nwg = (p.m + rows - 1) / rows;
+      if (used + nwg > resident) flush();
+      XPanelProb q{};
+      xpanel_carve(false, B->at<char>(B->o_xp) + p.inst * xpanel_bytes(false), &q.p);
+      q.p.A = p.A; q.p.ipiv = p.ipiv; q.p.lda = p.lda; q.p.m = p.m; q.p.w = NB; q.p.piv_off = p.piv_off; q.p.nwg = nwg;
+      q.p.err = B->flags() + 2 * p.inst;
+      q.p.seq0 = 1 + p.piv_off;      // the exchange memory is cleared before each factorisation
+      q.blk0 = used;
+      chunk.push_back(q);
+      used += nwg;
+    }
+    flush();
+    return BFA_OK;
+  }
+
   int lu()
   {
     int maxNp = 0;
@@ -651,7 +692,11 @@ struct Planner {
         const int64_t ld = B->Np[i];
         ps.push_back({A + (size_t)j * ld + j, ld, B->Np[i] - j, B->ipiv(i) + j, j, i});
       }
-      int rc = panel_rec(ps, NB);
+      std::vector<Pan> tall, low;
+      for (const Pan &p : ps) (p.m > xpanel_max_rows(false) ? tall : low).push_back(p);
+      int rc = BFA_OK;
+      if (!tall.empty()) rc = panel_rec(tall, NB);
+      if (!rc && !low.empty()) rc = panel_regs(low);
       if (rc) return rc;
       std::vector<SwapProb> sw;
       std::vector<c2 *> Bm;
@@ -664,7 +709,10 @@ struct Planner {
         const int *ip = B->ipiv(i);
         SwapProb s{};
         s.A = A; s.ipiv = ip; s.lda = p.lda; s.c0 = 0; s.c1 = j; s.k0 = j; s.kb = NB;
+        // a register panel leaves its multipliers in the rows of their step
+        if (p.m <= xpanel_max_rows(false)) { s.own = 1; s.c1 = j + NB; }
         sw.push_back(s);
+        s.own = 0;
         s.c0 = j + NB; s.c1 = B->Np[i];
         sw.push_back(s);
         const int rest = B->Np[i] - j - NB;
@@ -903,8 +951,11 @@ int build_plan(bfa_batch *B, double tol, int maxit)
   unsigned *cnt = B->counters();
   int *flags0 = B->flags();
   const size_t nflags = (size_t)2 * ni;
-  P.op([cnt, ncnt, flags0, nflags](hipStream_t st) {
+  unsigned *xp = B->at<unsigned>(B->o_xp);
+  const size_t nxp = ni * xpanel_bytes(false) / 4;
+  P.op([cnt, ncnt, flags0, nflags, xp, nxp](hipStream_t st) {
     hipLaunchKernelGGL(k_fill_u32, dim3(64), dim3(256), 0, st, cnt, ncnt);
+    hipLaunchKernelGGL(k_fill_u32, dim3(512), dim3(256), 0, st, xp, nxp);
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, (unsigned *)flags0, nflags);
   });
   P.op([B, o_sol, ni, scol](hipStream_t st) {
@@ -939,7 +990,7 @@ int build_plan(bfa_batch *B, double tol, int maxit)
       hipLaunchKernelGGL(kg_refine_check, dim3(ni), dim3(64), 0, st, d, ni, npw, tol);
     });
   }
-  // --- power (the complex64 LU storage becomes the EMT scratch)
+  // --- power
   P.phase = 3;
   P.op([B, o_emt, ni, nemt, nrow, fs, pws, npw](hipStream_t st) {
     const AsmInst *d = dp<AsmInst>(B, o_emt);
@@ -1034,6 +1085,7 @@ extern "C" int bfa_batch_create(int count, bfa_geometry *const *geoms, const bfa
   B->o_resid = take((size_t)count * 8);
   B->o_flags = take((size_t)count * 8);
   B->o_counters = take(B->ncounters_max * CSTRIDE * 4);
+  B->o_xp = take(count * xpanel_bytes(false));
   B->o_hist_it = take((size_t)BATCH_MAXFREQ * count * 4);
   B->o_hist_res = take((size_t)BATCH_MAXFREQ * count * 8);
   B->o_hist_info = take((size_t)BATCH_MAXFREQ * count * 4);

@@ -31,13 +31,13 @@ struct TrsmProb {
   int kb, n, blk0, pad;
 };
 
-// rows k0..k0+kb-1 <-> ipiv[.] on columns [c0, c1) of A; 128 columns per
-// workgroup from blk0
+// rows k0..k0+kb-1 <-> ipiv[.] on columns [c0, c1) of A (own: on column
+// c >= k0 only those after c); 128 columns per workgroup from blk0
 struct SwapProb {
   void *A;
   const int *ipiv;
   int64_t lda;
-  int c0, c1, k0, kb, blk0, pad;
+  int c0, c1, k0, kb, blk0, own;
 };
 
 // Panel workspace of one problem (cross-workgroup slots and barrier)

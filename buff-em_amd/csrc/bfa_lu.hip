@@ -1017,7 +1017,10 @@ __global__ __launch_bounds__(128) void kg_swap(const SwapProb *__restrict__ d, i
 {
   const SwapProb q = d[find_prob(d, np, blockIdx.x)];
   const int c = q.c0 + (blockIdx.x - q.blk0) * 128 + threadIdx.x;
-  if (c < q.c1) laswp_col<T>((cplx<T> *)q.A, q.lda, c, q.k0, q.kb, q.ipiv);
+  if (c >= q.c1) return;
+  // own: the columns of the panel itself take the interchanges after theirs
+  const int skip = q.own ? max(0, c - q.k0 + 1) : 0;
+  laswp_col<T>((cplx<T> *)q.A, q.lda, c, q.k0 + skip, q.kb - skip, q.ipiv);
 }
 
 template <typename T>
@@ -1066,12 +1069,12 @@ static int lu_work(LUWork *&w)
   HIPCHECK(hipGetDeviceProperties(&prop, dev));
   w->num_cu = prop.multiProcessorCount;
   w->maxwg = 1024;
-  const size_t bytes = 2 * (size_t)w->maxwg * PW * 16 + 2 * PW * 16 + 2 * PB_WORDS * 4 + 64 + xpanel_bytes();
+  const size_t bytes = 2 * (size_t)w->maxwg * PW * 16 + 2 * PW * 16 + 2 * PB_WORDS * 4 + 64 + xpanel_bytes(true);
   HIPCHECK(hipMalloc(&w->mem, bytes));
   HIPCHECK(hipMemset(w->mem, 0, bytes));
   char *p = (char *)w->mem;
-  xpanel_carve(p, &w->xp);
-  p += xpanel_bytes();
+  xpanel_carve(true, p, &w->xp);
+  p += xpanel_bytes(true);
   w->pw.rowdata = p; p += 2 * (size_t)w->maxwg * PW * 16;
   w->pw.rowj = p; p += 2 * PW * 16;
   w->bars = (unsigned *)p;                       // two sets of PB_WORDS, both zero
@@ -1196,7 +1199,7 @@ static int panel_regs(cplx<T> *A, int m, int w, int64_t lda, int *ipiv, int piv_
 {
   if (lw->xseq + w >= 1u << 24) {
     // stale words must not look current: rows and flags restart from zero
-    const int nw = (int)(xpanel_bytes() / 4);
+    const int nw = (int)(xpanel_bytes(true) / 4);
     hipLaunchKernelGGL(k_zero_u32, dim3((nw + 255) / 256), dim3(256), 0, st, (unsigned *)lw->xp.data, nw);
     lw->xseq = 1;
   }

@@ -21,8 +21,20 @@ struct XPanel {
   unsigned seq0;         // this launch's first sequence number (24 bits, w of them used)
   int m, w, piv_off, nwg;
 };
-size_t xpanel_bytes();
-void xpanel_carve(char *mem, XPanel *p);
+// exchange memory of one panel at a time: bytes, and its division
+size_t xpanel_bytes(bool f64);
+void xpanel_carve(bool f64, char *mem, XPanel *p);
 int xpanel_max_rows(bool f64);
 int launch_xpanel(bool f64, XPanel p, hipStream_t st);
+
+// several complex64 panels in one launch, XPanelProb::p.nwg workgroups each
+// from blk0; rows: rows a workgroup, one of xpanel_group_rows' values
+struct XPanelProb {
+  XPanel p;
+  int blk0, pad;
+};
+// rows a workgroup for panels of at most m rows that fill `total` rows in all,
+// and the workgroups that may run at once with it (0: none)
+int xpanel_group_rows(int m, int64_t total, int *resident);
+void launch_xpanel_g(const XPanelProb *d, int np, int nblk, int rows, hipStream_t st);
 }  // namespace bfa

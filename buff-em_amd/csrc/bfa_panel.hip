@@ -151,7 +151,7 @@ template <int LO, int HI, typename T, int R> __device__ __forceinline__ void reg
 }
 
 #define XP_NT 256
-#define XP_SPIN_LIMIT (1u << 22)
+#define XP_SPIN_LIMIT (1u << 24)
 
 template <typename T, int NR> struct XpShared { zc<T> col[4][NR]; };
 
@@ -403,6 +403,33 @@ template <typename T, int WB, int R> __global__ __launch_bounds__(XP_NT) void k_
   xpanel_body<T, WB, R>(p, blockIdx.x, sh);
 }
 
+// grouped: workgroups blk0 .. blk0 + nwg - 1 of the launch factor panel d[i]
+template <int R> __global__ __launch_bounds__(XP_NT) void kg_xpanel(const XPanelProb *__restrict__ d, int np)
+{
+  __shared__ XpShared<float, R> sh;
+  int lo = 0, hi = np - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (d[mid].blk0 <= (int)blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  xpanel_body<float, 256, R>(d[lo].p, blockIdx.x - d[lo].blk0, sh);
+}
+
+template <int R> int resident_g()
+{
+  static int n = -1;
+  if (n < 0) {
+    int per = 0, dev = 0;
+    hipDeviceProp_t prop;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kg_xpanel<R>, XP_NT, 0) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
+      per = 0;
+    n = per > 0 ? std::min(per, 2) * prop.multiProcessorCount : 0;
+  }
+  return n;
+}
+
 template <typename T, int WB, int R> void launch(XPanel p, hipStream_t st)
 {
   p.nwg = (p.m + XP_NT / WB * R - 1) / (XP_NT / WB * R);
@@ -412,13 +439,13 @@ template <typename T, int WB, int R> void launch(XPanel p, hipStream_t st)
 }  // namespace
 
 namespace bfa {
-static const size_t kRowBytes = (size_t)XP_NBUF * (XP_MAXWG + 1) * XP_PLANE * 32;
-size_t xpanel_bytes() { return kRowBytes + (size_t)XP_NBUF * XP_MAXWG * XP_FSTRIDE * 8; }
+static size_t row_bytes(bool f64) { return (size_t)XP_NBUF * (XP_MAXWG + 1) * XP_PLANE * (f64 ? 32 : 16); }
+size_t xpanel_bytes(bool f64) { return row_bytes(f64) + (size_t)XP_NBUF * XP_MAXWG * XP_FSTRIDE * 8; }
 
-void xpanel_carve(char *mem, XPanel *p)
+void xpanel_carve(bool f64, char *mem, XPanel *p)
 {
   p->data = mem;
-  p->flags = (unsigned long long *)(mem + kRowBytes);
+  p->flags = (unsigned long long *)(mem + row_bytes(f64));
 }
 
 // Rows a workgroup holds, fewest first: a column's time grows with them (the
@@ -446,5 +473,28 @@ int launch_xpanel(bool f64, XPanel p, hipStream_t st)
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? BFA_OK : fail(BFA_ERR_HIP, "register panel launch: %s", hipGetErrorString(e));
+}
+
+// Fewest rows that keep the launch to two workgroups a CU (a column's time
+// grows with the rows, see above, and with a second round of launches more)
+int xpanel_group_rows(int m, int64_t total, int *resident)
+{
+  const int rows[3] = {16, 32, 48}, res[3] = {resident_g<16>(), resident_g<32>(), resident_g<48>()};
+  int pick = -1;
+  for (int i = 0; i < 3; i++) {
+    if (m > rows[i] * XP_MAXWG || res[i] < XP_MAXWG) continue;
+    pick = i;
+    if (total <= (int64_t)rows[i] * res[i]) break;
+  }
+  *resident = pick < 0 ? 0 : res[pick];
+  return pick < 0 ? 0 : rows[pick];
+}
+
+void launch_xpanel_g(const XPanelProb *d, int np, int nblk, int rows, hipStream_t st)
+{
+  if (nblk <= 0) return;
+  if (rows == 16) hipLaunchKernelGGL(kg_xpanel<16>, dim3(nblk), dim3(XP_NT), 0, st, d, np);
+  else if (rows == 32) hipLaunchKernelGGL(kg_xpanel<32>, dim3(nblk), dim3(XP_NT), 0, st, d, np);
+  else hipLaunchKernelGGL(kg_xpanel<48>, dim3(nblk), dim3(XP_NT), 0, st, d, np);
 }
 }  // namespace bfa
