@@ -18,6 +18,7 @@
 //   AssembleRHSVector              src/libs/libbuff/RHSVector.cc:62-124
 //   GetEMTPFT                      src/libs/libbuff/EMTPFT.cc:85-546
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -131,6 +132,7 @@ extern "C" int bfa_geometry_upload(bfa_geometry *g, void *stream)
   // far-field tiles: distinct tetrahedra of each FT2-BF tile, in order of
   // first appearance, and the slot of every (BF, side) in that list
   const int nft = (N + FT2 - 1) / FT2;
+  g->ft_max = 0;
   std::vector<int> ftTab((size_t)nft * FTAB, -1);
   for (int tile = 0; tile < nft; tile++) {
     int *row = &ftTab[(size_t)tile * FTAB];
@@ -145,6 +147,7 @@ extern "C" int bfa_geometry_upload(bfa_geometry *g, void *stream)
       row[2 * FT2 + k] = u;
     }
     row[4 * FT2] = n;
+    g->ft_max = std::max(g->ft_max, n);
   }
   for (int t = 0; t < nt; t++) {
     volcen[t] = g->tetVol[t];
@@ -658,7 +661,7 @@ __device__ __forceinline__ void tp_point_pair(const double *x, const double *y, 
   const double R0 = x[0] - y[0], R1 = x[1] - y[1], R2 = x[2] - y[2];
   const double r2 = R0 * R0 + R1 * R1 + R2 * R2, ir = rsqrt_nr(r2), r = r2 * ir;
   double sn, co;
-  sincos(kre * r, &sn, &co);
+  sincos_mod(kre * r, &sn, &co);
   double amp = x[3] * y[3] * ir;
   if (!REALK) amp *= exp(-kim * r);
   const double gr = amp * co, gi = amp * sn;
@@ -748,7 +751,7 @@ __device__ __forceinline__ SplitK split_setup(const double *cS, const double *cT
   const double D2 = d0 * d0 + d1 * d1 + d2 * d2, iD = rsqrt_nr(D2), D = D2 * iD;
   z.e0 = d0 * iD; z.e1 = d1 * iD; z.e2 = d2 * iD; z.D = D; z.hiD = 0.5 * iD;
   double sn, co;
-  sincos(kre * D, &sn, &co);
+  sincos_mod(kre * D, &sn, &co);
   double amp = iD;
   if (!REALK) amp *= exp(-kim * D);
   z.g0r = amp * co; z.g0i = amp * sn;
@@ -1068,149 +1071,199 @@ __global__ __launch_bounds__(TPT_THREADS) void k_tp_table(DevGeom g, double kre,
   tp_table_tile<REALK, SPLIT>(g, kre, kim, tab, bs, bt, sh);
 }
 
-// the 16 moments of row tetrahedron S and column tetrahedron T from the table
-__device__ __forceinline__ void tp_fetch(const double *__restrict__ tab, int S, int T, int nt, double *m)
-{
-  const bool sw = S > T;
-  const double2 *r = (const double2 *)(tab + (sw ? tp_index(T, S, nt) : tp_index(S, T, nt)) * 16);
-  double v[16];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const double2 x = r[i];
-    v[2 * i] = x.x;
-    v[2 * i + 1] = x.y;
-  }
-#pragma unroll
-  for (int i = 0; i < 16; i++) {
-    // I0 (0, 1) and Ixy (14, 15) stay; Ix (2..7) and Iy (8..13) exchange
-    const int src = (i >= 2 && i < 14 && sw) ? (i < 8 ? i + 6 : i - 6) : i;
-    m[i] = v[src];
-  }
-}
-
-// Pass 2: the single pass's tile with the moments read from the table
-// instead of evaluated, and the tile's 64 BFs (prefactors, Q minus the
-// centroid of each side's tetrahedron, vertices) read once into LDS by field
-// (11.8 ms at N = 19,872; 12.4 ms reading them per BF pair).  Slower
-// variants measured: eight lanes per record (16.2 ms), results staged in
-// LDS for coalesced stores of both triangles (13.3 ms), the BF data in LDS
-// by BF (15.5 ms: bank conflicts), 26 KB of LDS with the records read per
-// BF pair (15.8 ms), the tiles dealt to the XCDs in contiguous runs that
-// walk two tile rows at a time, so that neighbouring tiles sharing records
-// run on one L2 (fetch 25 -> 16 GB per launch, time 12.2 -> 12.4 ms), one
-// workgroup per CU looping over the tiles (so that stores drain while the
-// next tile loads; unchanged) -- the tile is bound by the latency of its
-// dependent global reads, not by HBM (without the table reads it still
-// takes 10.7 ms).
-// LDS of one pass-2 tile: the records, and the tile's BFs by field
-struct GatherShared {
-  FarTpShared t;
-  double bfd[2][8][FT2];
-  int bfv[2][5][FT2];
+// Pass 2: a 32 x 32 BF tile combines the table's records in two steps.  A BF
+// pair's element is a sum over its four tetrahedron pairs (S, T) of
+//   pf_a pf_b [Ixy - b.Ix - a.Iy + (a.b) I0 - 9 I0/k^2],
+// so for a row tetrahedron S and a column BF the sum over the BF's two T is
+//   s - a.v,  s = sum pf_b [Ixy - b.Ix - 9 I0/k^2],  v = sum pf_b [Iy - b I0],
+// four complex numbers that every row BF on S shares: 992 + 2,048 short
+// combinations a tile instead of 4,096 long ones, and a quarter of the LDS
+// reads.  Row tetrahedra go through LDS four at a time (records, then s and
+// v; the next four's records are on their way meanwhile), so a workgroup holds
+// 35 KB of LDS, not the tile's 151 KB of records, and four share a CU.
+// N = 19,872: 11.8 -> 5.4 ms (before: one workgroup a CU, all of a tile's
+// records in LDS, bound by the latency of its dependent phases).  Tried on
+// top of it: tiles dealt to the XCDs in bands that share records, 6.1 -> 6.3
+// ms at the time -- the records' traffic is not the bound, issue is.
+#define GS_CH 4            // row tetrahedra at a time
+#define GS_NT 256
+typedef double dv2 __attribute__((ext_vector_type(2)));
+template <int NC> struct GatherShared {
+  dv2 rec[GS_CH][NC][9];       // a record's 8 entries, padded: lanes on consecutive tetrahedra read distinct banks
+  double H[GS_CH][8][FT2];         // s, v (re, im) of each column BF
+  int rt[2 * FT2], ct[2 * FT2];    // distinct tetrahedra
+  double rpf[2][FT2], ral[2][3][FT2];
+  int rslot[2][FT2], rv[5][FT2], cv[5][FT2];
 };
 
+// x plus the other half-wave's x
+__device__ __forceinline__ double half_sum(double x)
+{
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+
+template <int NC>
 __device__ __forceinline__ void far_gather_tile(const DevGeom &g, double kre, double kim,
                                                 const double *__restrict__ tpt, cd *M, int64_t ld, int ti, int tj,
-                                                GatherShared &gs)
+                                                GatherShared<NC> &sh)
 {
-  FarTpShared &sh = gs.t;
-  double (&bfd)[2][8][FT2] = gs.bfd;
-  int (&bfv)[2][5][FT2] = gs.bfv;
-  const int tid = threadIdx.x, nth = blockDim.x, N = g.nbf, nt = g.nt;
-  const int *tab[2] = {g.ftTab + (size_t)ti * FTAB, g.ftTab + (size_t)tj * FTAB};
-  const int nr = tab[0][4 * FT2], nc = tab[1][4 * FT2];
-  for (int idx = tid; idx < 2 * 2 * FT2; idx += nth) {
-    const int which = idx / (2 * FT2), k = idx % (2 * FT2);
-    sh.slot[which][k] = tab[which][2 * FT2 + k];
+  const int tid = threadIdx.x, lane = tid & 63, N = g.nbf, nt = g.nt;
+  const int *rtab = g.ftTab + (size_t)ti * FTAB, *ctab = g.ftTab + (size_t)tj * FTAB;
+  const int nr = rtab[4 * FT2], nc = ctab[4 * FT2];
+  const double *tetCen = g.tetVol + nt;
+  // this thread's column BF and side (one wave: 32 BFs x 2 sides)
+  const int lb = tid & 31, sb = (tid >> 5) & 1, b = tj * FT2 + lb;
+  const int cslot = ctab[2 * FT2 + 2 * lb + sb];
+  double pfb = 0.0, be[3] = {0.0, 0.0, 0.0};
+  if (b < N) {
+    const int T = g.bfT[2 * b + sb];
+    pfb = g.bfPF[2 * b + sb];
+#pragma unroll
+    for (int d = 0; d < 3; d++) be[d] = g.bfQ[6 * b + 3 * sb + d] - tetCen[3 * T + d];
   }
-  for (int idx = tid; idx < 2 * 2 * FT2 * 16; idx += nth) {
-    const int which = idx / (2 * FT2 * 16), rem = idx % (2 * FT2 * 16);
-    const int u = rem / 16, e = rem % 16;
-    if (u < (which ? nc : nr)) sh.pts[which][e][u] = g.q4[(size_t)tab[which][u] * 16 + e];
-  }
-  __syncthreads();
-  for (int idx = tid; idx < 2 * 2 * FT2; idx += nth) {
-    const int which = idx / (2 * FT2), u = idx % (2 * FT2);
-    if (u < (which ? nc : nr))
-      for (int d = 0; d < 3; d++)
-        sh.cen[which][d][u] = 0.25 * (sh.pts[which][d][u] + sh.pts[which][4 + d][u] + sh.pts[which][8 + d][u] +
-                                      sh.pts[which][12 + d][u]);
-  }
-  __syncthreads();
-  for (int idx = tid; idx < 2 * FT2; idx += nth) {
-    const int which = idx / FT2, k = idx % FT2;
-    const int a = (which ? tj : ti) * FT2 + k;
-    if (a >= N) continue;
-    for (int v = 0; v < 5; v++) bfv[which][v][k] = g.bfV[5 * a + v];
-    for (int sd = 0; sd < 2; sd++) {
-      const int u = sh.slot[which][2 * k + sd];
-      bfd[which][4 * sd][k] = g.bfPF[2 * a + sd];
-      for (int d = 0; d < 3; d++) bfd[which][4 * sd + 1 + d][k] = g.bfQ[6 * a + 3 * sd + d] - sh.cen[which][d][u];
+  if (tid < 4 * FT2) {
+    const int side = tid / (2 * FT2), u = tid % (2 * FT2);
+    const int t = u < (side ? nc : nr) ? (side ? ctab : rtab)[u] : 0;
+    (side ? sh.ct : sh.rt)[u] = t;
+  } else if (tid < 6 * FT2) {
+    const int k = tid - 4 * FT2, la = k >> 1, sa = k & 1, a = ti * FT2 + la;
+    sh.rslot[sa][la] = rtab[2 * FT2 + k];
+    double pf = 0.0, al[3] = {0.0, 0.0, 0.0};
+    if (a < N) {
+      const int S = g.bfT[2 * a + sa];
+      pf = g.bfPF[2 * a + sa];
+#pragma unroll
+      for (int d = 0; d < 3; d++) al[d] = g.bfQ[6 * a + 3 * sa + d] - tetCen[3 * S + d];
     }
-  }
-  const bool direct = nr * nc > FTT_MAX;
-  if (!direct) {
-    for (int pidx = tid; pidx < nr * nc; pidx += nth) {
-      double m[16];
-      tp_fetch(tpt, tab[0][pidx / nc], tab[1][pidx % nc], nt, m);
+    sh.rpf[sa][la] = pf;
 #pragma unroll
-      for (int i = 0; i < 16; i++) sh.mom[i][pidx] = m[i];
-    }
+    for (int d = 0; d < 3; d++) sh.ral[sa][d][la] = al[d];
+  } else if (tid < 7 * FT2) {
+    const int la = tid - 6 * FT2, a = ti * FT2 + la;
+#pragma unroll
+    for (int v = 0; v < 5; v++) sh.rv[v][la] = a < N ? g.bfV[5 * a + v] : -2;
+  } else {
+#pragma unroll
+    for (int v = 0; v < 5; v++) sh.cv[v][lb] = b < N ? g.bfV[5 * b + v] : -1;
   }
   __syncthreads();
-  const double k2re = kre * kre - kim * kim, k2im = 2.0 * kre * kim;
-  const double ik2d = k2re * k2re + k2im * k2im;
-  const double ik2re = k2re / ik2d, ik2im = -k2im / ik2d;
-  for (int pidx = tid; pidx < FT2 * FT2; pidx += nth) {
-    const int lb = pidx % FT2, la = pidx / FT2;
-    const int a = ti * FT2 + la, b = tj * FT2 + lb;
-    if (a >= N || b >= N || b < a) continue;
-    int va[5], vb[5];
+  const double k2re = kre * kre - kim * kim, k2im = 2.0 * kre * kim, ik2d = k2re * k2re + k2im * k2im;
+  const double q9re = 9.0 * k2re / ik2d, q9im = -9.0 * k2im / ik2d;        // 9 / k^2
+  const int a0 = (tid >> 5) * 4;                   // this thread's four row BFs
+  int slot[2][4];
 #pragma unroll
-    for (int v = 0; v < 5; v++) { va[v] = bfv[0][v][la]; vb[v] = bfv[1][v][lb]; }
-    if (bf_ncv(va, vb) > 0) continue;
-    double accr = 0.0, acci = 0.0;
+  for (int sa = 0; sa < 2; sa++)
 #pragma unroll
-    for (int sa = 0; sa < 2; sa++) {
-      const int us = sh.slot[0][2 * la + sa];
-      const double pfa = bfd[0][4 * sa][la], al0 = bfd[0][4 * sa + 1][la], al1 = bfd[0][4 * sa + 2][la],
-                   al2 = bfd[0][4 * sa + 3][la];
+    for (int i = 0; i < 4; i++) slot[sa][i] = sh.rslot[sa][a0 + i];
+  cd acc[4];
 #pragma unroll
-      for (int sb = 0; sb < 2; sb++) {
-        const int ut = sh.slot[1][2 * lb + sb];
-        const double pfb = bfd[1][4 * sb][lb], be0 = bfd[1][4 * sb + 1][lb], be1 = bfd[1][4 * sb + 2][lb],
-                     be2 = bfd[1][4 * sb + 3][lb];
-        double m[16];
-        if (direct) {
-          tp_fetch(tpt, tab[0][us], tab[1][ut], nt, m);
-        } else {
+  for (int i = 0; i < 4; i++) acc[i] = {0.0, 0.0};
+  // records of row tetrahedra s0 .. s0 + 3, one a wave, eight threads a
+  // record; for S > T the record of (T, S), with Ix and Iy exchanged.  Record
+  // numbers fit 32 bits (2^32 of them would fill 550 GB).
+  constexpr int NL = NC / 8;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), e = tid & 7, u0 = (tid >> 3) & 7;
+  const int ex = e >= 1 && e <= 3 ? e + 3 : e >= 4 && e <= 6 ? e - 3 : e;
+  int T[NL];
+  unsigned tbase[NL];                              // row T's first record, less T
 #pragma unroll
-          for (int i = 0; i < 16; i++) m[i] = sh.mom[i][us * nc + ut];
-        }
-        const double ab = al0 * be0 + al1 * be1 + al2 * be2;
-        double dr = m[14] - (be0 * m[2] + be1 * m[4] + be2 * m[6]) - (al0 * m[8] + al1 * m[10] + al2 * m[12]) + ab * m[0];
-        double di = m[15] - (be0 * m[3] + be1 * m[5] + be2 * m[7]) - (al0 * m[9] + al1 * m[11] + al2 * m[13]) + ab * m[1];
-        dr -= 9.0 * (m[0] * ik2re - m[1] * ik2im);
-        di -= 9.0 * (m[0] * ik2im + m[1] * ik2re);
-        const double f = pfa * pfb;
-        accr += f * dr;
-        acci += f * di;
+  for (int k = 0; k < NL; k++) {
+    T[k] = sh.ct[u0 + 8 * k];
+    tbase[k] = (unsigned)((int64_t)T[k] * nt - (int64_t)T[k] * (T[k] + 1) / 2);
+  }
+  dv2 pre[NL];
+  auto fetch = [&](int s0) __attribute__((always_inline)) {
+    const int S = __builtin_amdgcn_readfirstlane(sh.rt[min(s0 + wv, 2 * FT2 - 1)]);
+    const unsigned sbase = (unsigned)((int64_t)S * nt - (int64_t)S * (S + 1) / 2);
+#pragma unroll
+    for (int k = 0; k < NL; k++) {
+      const bool sw = S > T[k];
+      const unsigned row = sw ? tbase[k] + S : sbase + T[k];
+      pre[k] = ((const dv2 *)tpt)[(size_t)row * 8 + (sw ? ex : e)];
+    }
+  };
+  fetch(0);
+#pragma unroll 1
+  for (int s0 = 0; s0 < nr; s0 += GS_CH) {
+#pragma unroll
+    for (int k = 0; k < NL; k++) sh.rec[wv][u0 + 8 * k][e] = pre[k];
+    __syncthreads();
+    if (s0 + GS_CH < nr) fetch(s0 + GS_CH);
+    // s and v of wave `si`'s row tetrahedron: one side a thread, the two added across the wave's halves
+    {
+      const int si = tid >> 6;
+      double h[8];
+      const dv2 *m = sh.rec[si][cslot];
+      const dv2 i0 = m[0], xy = m[7];
+      double sr = xy.x - (i0.x * q9re - i0.y * q9im), sm = xy.y - (i0.x * q9im + i0.y * q9re);
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const dv2 ix = m[1 + d], iy = m[4 + d];
+        sr -= be[d] * ix.x;
+        sm -= be[d] * ix.y;
+        h[2 + 2 * d] = pfb * (iy.x - be[d] * i0.x);
+        h[3 + 2 * d] = pfb * (iy.y - be[d] * i0.y);
+      }
+      h[0] = pfb * sr;
+      h[1] = pfb * sm;
+#pragma unroll
+      for (int i = 0; i < 8; i++) h[i] = half_sum(h[i]);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const double lo = h[i], hi = h[4 + i];
+        sh.H[si][4 * sb + i][lb] = sb ? hi : lo;
       }
     }
-    const cd v = {accr / FOURPI, acci / FOURPI};
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int sa = 0; sa < 2; sa++) {
+        const int u = slot[sa][i] - s0;
+        if (u < 0 || u >= GS_CH) continue;
+        const double pf = sh.rpf[sa][a0 + i];
+        double re = sh.H[u][0][lb], im = sh.H[u][1][lb];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          const double al = sh.ral[sa][d][a0 + i];
+          re -= al * sh.H[u][2 + 2 * d][lb];
+          im -= al * sh.H[u][3 + 2 * d][lb];
+        }
+        acc[i].re += pf * re;
+        acc[i].im += pf * im;
+      }
+  }
+  int vb[5];
+#pragma unroll
+  for (int v = 0; v < 5; v++) vb[v] = sh.cv[v][lb];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int a = ti * FT2 + a0 + i;
+    if (a >= N || b >= N || b < a) continue;
+    int va[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) va[v] = sh.rv[v][a0 + i];
+    if (bf_ncv(va, vb) > 0) continue;
+    const cd v = {acc[i].re * (1.0 / FOURPI), acc[i].im * (1.0 / FOURPI)};
     M[(size_t)b * ld + a] = v;
     M[(size_t)a * ld + b] = v;
   }
 }
 
-__global__ __launch_bounds__(FT_THREADS) void k_far_gather(DevGeom g, double kre, double kim,
-                                                           const double *__restrict__ tpt, cd *M, int64_t ld,
-                                                           int ntiles)
+// NC: most distinct tetrahedra of a tile (31 on average on the Kuhn spheres,
+// 34 at most; 64 is any mesh's bound)
+template <int NC>
+__global__ __launch_bounds__(GS_NT, 4) void k_far_gather(DevGeom g, double kre, double kim,
+                                                      const double *__restrict__ tpt, cd *M, int64_t ld, int ntiles)
 {
-  __shared__ GatherShared gs;
+  __shared__ GatherShared<NC> sh;
   int ti, tj;
   tile_coords(blockIdx.x, ntiles, ti, tj);
-  far_gather_tile(g, kre, kim, tpt, M, ld, ti, tj, gs);
+  far_gather_tile<NC>(g, kre, kim, tpt, M, ld, ti, tj, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -1766,8 +1819,12 @@ static int assemble_vie(bfa_geometry *g, double omega_re, double omega_im, const
       if (rk) hipLaunchKernelGGL((k_tp_table<true, false>), gr1, bl1, 0, st, g->dg, omega_re, 0.0, tpt, ntb);
       else hipLaunchKernelGGL((k_tp_table<false, false>), gr1, bl1, 0, st, g->dg, omega_re, omega_im, tpt, ntb);
     }
-    hipLaunchKernelGGL(k_far_gather, dim3((unsigned)nblk2), dim3(FT_THREADS), 0, st, g->dg, omega_re, omega_im,
-                       (const double *)tpt, M, ld, nt2);
+    if (g->ft_max <= 40)
+      hipLaunchKernelGGL(k_far_gather<40>, dim3((unsigned)nblk2), dim3(GS_NT), 0, st, g->dg, omega_re, omega_im,
+                         (const double *)tpt, M, ld, nt2);
+    else
+      hipLaunchKernelGGL(k_far_gather<64>, dim3((unsigned)nblk2), dim3(GS_NT), 0, st, g->dg, omega_re, omega_im,
+                         (const double *)tpt, M, ld, nt2);
   } else {
     const dim3 gr2((unsigned)nblk2), bl2(FT_THREADS);
     if (far32) {
@@ -2319,13 +2376,14 @@ __global__ __launch_bounds__(TPT_THREADS) void kg_tp_table(const AsmInst *__rest
   tp_table_tile<REALK, false>(q.g, fs->omega_re, REALK ? 0.0 : fs->omega_im, q.tpt, bs, bt, sh);
 }
 
-__global__ __launch_bounds__(FT_THREADS) void kg_far_gather(const AsmInst *__restrict__ d, int ni, const FreqState *fs)
+template <int NC>
+__global__ __launch_bounds__(GS_NT, 4) void kg_far_gather(const AsmInst *__restrict__ d, int ni, const FreqState *fs)
 {
-  __shared__ GatherShared gs;
+  __shared__ GatherShared<NC> sh;
   const AsmInst &q = d[find_inst(d, ni, blockIdx.x, GF_FAR)];
   int ti, tj;
   tile_coords(blockIdx.x - q.far0, q.ntiles, ti, tj);
-  far_gather_tile(q.g, fs->omega_re, fs->omega_im, q.tpt, (cd *)q.M, q.ldm, ti, tj, gs);
+  far_gather_tile<NC>(q.g, fs->omega_re, fs->omega_im, q.tpt, (cd *)q.M, q.ldm, ti, tj, sh);
 }
 
 // EXPR: some instance's material is a compiled SVTensor (as k_near)
@@ -2384,9 +2442,11 @@ void launch_tp_table_g(const AsmInst *d, int ni, int ntab, const FreqState *fs, 
   else hipLaunchKernelGGL(kg_tp_table<false>, dim3(ntab), dim3(TPT_THREADS), 0, st, d, ni, fs);
 }
 
-void launch_far_gather_g(const AsmInst *d, int ni, int nfar, const FreqState *fs, hipStream_t st)
+void launch_far_gather_g(const AsmInst *d, int ni, int nfar, int ft_max, const FreqState *fs, hipStream_t st)
 {
-  if (nfar > 0) hipLaunchKernelGGL(kg_far_gather, dim3(nfar), dim3(FT_THREADS), 0, st, d, ni, fs);
+  if (nfar <= 0) return;
+  if (ft_max <= 40) hipLaunchKernelGGL(kg_far_gather<40>, dim3(nfar), dim3(GS_NT), 0, st, d, ni, fs);
+  else hipLaunchKernelGGL(kg_far_gather<64>, dim3(nfar), dim3(GS_NT), 0, st, d, ni, fs);
 }
 
 size_t tp_table_bytes(int nt) { return (size_t)nt * (nt + 1) / 2 * 16 * sizeof(double); }

@@ -933,7 +933,11 @@ int build_plan(bfa_batch *B, double tol, int maxit)
   // omega_im = 0), so the far field runs its real-k kernel
   if (B->tp_state == 1) {
     P.op([B, o_asm, ni, ntab, fs](hipStream_t st) { launch_tp_table_g(dp<AsmInst>(B, o_asm), ni, ntab, fs, true, st); });
-    P.op([B, o_asm, ni, nfar, fs](hipStream_t st) { launch_far_gather_g(dp<AsmInst>(B, o_asm), ni, nfar, fs, st); });
+    int ft_max = 0;
+    for (const bfa_geometry *g : B->geo) ft_max = std::max(ft_max, g->ft_max);
+    P.op([B, o_asm, ni, nfar, ft_max, fs](hipStream_t st) {
+      launch_far_gather_g(dp<AsmInst>(B, o_asm), ni, nfar, ft_max, fs, st);
+    });
   } else {
     P.op([B, o_asm, ni, nfar, fs](hipStream_t st) { launch_far_g(dp<AsmInst>(B, o_asm), ni, nfar, fs, true, st); });
   }

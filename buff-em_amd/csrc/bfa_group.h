@@ -131,7 +131,8 @@ void launch_far_g(const AsmInst *d, int ni, int nblk, const FreqState *fs, bool 
 // the two-pass far field of the instances (every tpt set): the moment tables
 // (ntab workgroups in all), then the BF tiles gathering them (nfar)
 void launch_tp_table_g(const AsmInst *d, int ni, int ntab, const FreqState *fs, bool realk, hipStream_t st);
-void launch_far_gather_g(const AsmInst *d, int ni, int nfar, const FreqState *fs, hipStream_t st);
+// ft_max: most distinct tetrahedra of any instance's tile
+void launch_far_gather_g(const AsmInst *d, int ni, int nfar, int ft_max, const FreqState *fs, hipStream_t st);
 // bytes of one instance's moment table (nt tetrahedra)
 size_t tp_table_bytes(int nt);
 // expr: some instance's material is a compiled SVTensor (material kind 4)

@@ -83,6 +83,7 @@ struct bfa_geometry {
   int device = -1;
   bool uploaded = false, static_built = false;
   int td_order = 0;
+  int ft_max = 0;                             // most distinct tetrahedra of a far-field tile
   bfa::DevBuffers d;
   bfa::DevGeom dg{};
 };
