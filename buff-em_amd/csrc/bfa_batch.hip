@@ -303,7 +303,7 @@ struct bfa_batch {
   int tp_state = 0;              // 0 not tried, 1 tables, -1 single pass
   // everything else in one allocation; per-instance byte offsets
   void *small = nullptr;
-  struct Off { size_t ipiv, perm, B, X, R, D, Y, Xs, inv, tick, P, norms, part, emt, sdata, sj; };
+  struct Off { size_t ipiv, perm, B, X, R, D, Y, Xs, inv, tick, P, norms, part, emt, gram, sdata, sj; };
   std::vector<Off> off;
   size_t o_fs = 0, o_conv = 0, o_iters = 0, o_resid = 0, o_counters = 0, o_flags = 0;
   size_t o_xp = 0;               // register panels' exchange memory, xpanel_bytes(false) an instance
@@ -893,6 +893,7 @@ std::vector<AsmInst> asm_descs(const bfa_batch *B, bool solution, int &nfar, int
     q.B = solution ? (void *)B->Xp(i) : (void *)B->Bp(i);
     q.ldb = B->Np[i];
     q.Q = B->at<double>(B->off[i].emt);
+    q.gram = B->at<void>(B->off[i].gram);
     q.part = B->at<double>(B->off[i].part);
     const int N = B->N[i];
     q.ntiles = (N + FT2 - 1) / FT2;
@@ -1078,6 +1079,7 @@ extern "C" int bfa_batch_create(int count, bfa_geometry *const *geoms, const bfa
     f.norms = take((size_t)npw * nblk * 16);
     f.part = take((size_t)2 * npw * nblk * 8);
     f.emt = take(emt_work_doubles(geoms[i]->nt, npw) * 8);
+    f.gram = take((size_t)geoms[i]->nt * 256);
     f.sdata = take((size_t)2 * 256 * PWID * 16);
     f.sj = take(2 * PWID * 16);
     B->off.push_back(f);

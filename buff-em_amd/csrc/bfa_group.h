@@ -106,6 +106,7 @@ struct AsmInst {
   void *M;               // complex128 VIE matrix, N x N used, ld = ldm
   void *B;               // complex128 right-hand sides / solutions, ld = ldb
   double *Q;             // EMT work space (emt_work_doubles)
+  void *gram;            // [nt][4][4] complex Gram blocks
   double *part;          // EMT sums: [0][npw][0] scattered, [1][npw][row blocks] extinction
   int64_t ldm, ldb;
   int far0, ntiles;      // far-field tiles (upper triangle of FT2 x FT2 BF tiles) from far0

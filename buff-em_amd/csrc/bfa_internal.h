@@ -56,6 +56,7 @@ struct DevBuffers {
   void *table = nullptr;       // [nnz][6] FIBBI records
   void *tpTab = nullptr;       // far field: 16 moments per tetrahedron pair S <= T (per frequency)
   size_t tpTabBytes = 0;
+  void *gram = nullptr;        // [nt][4][4] complex Gram blocks (per frequency and material)
 };
 
 }  // namespace bfa
