@@ -1073,7 +1073,7 @@ extern "C" int bfa_batch_create(int count, bfa_geometry *const *geoms, const bfa
     f.D = take((size_t)npw * Np * 8);
     f.Y = take((size_t)npw * Np * 8);
     f.Xs = take((size_t)npw * Np * 8);
-    f.inv = take((size_t)2 * (Np / SVB) * SVB * SVB * 8);
+    f.inv = take((size_t)4 * (Np / SVB) * SVB * SVB * 8);
     f.tick = take(8);
     f.P = take((size_t)nchunk * npw * N * 16);
     f.norms = take((size_t)npw * nblk * 16);

@@ -51,21 +51,38 @@ __global__ void k_c2z_add(const c2 *D, int64_t ldd, z2 *X, int64_t ldx, int m, i
 }
 
 // Residual partials: P[chunk][j][r] = sum_{c in chunk} M(r, c) X(c, j).
-// Grid: (row blocks of 256, column chunks); one thread per row, M streamed
-// once, coalesced along rows; X for the chunk staged in LDS.
+// Grid: (row blocks of 256, column chunks, groups of RES_MAXRHS right-hand
+// sides); one thread per row, M streamed once a group, coalesced along rows; X
+// for the chunk staged in LDS.
 #define RES_CHUNK 256
 #define RES_MAXRHS 8
+// right-hand sides of one launch: bounds the partials at what a batch needs
+#define RES_BATCH 32
+
+// Columns of a chunk.  A thread walks its chunk serially, so what bounds a
+// small system is the length of the chunk and the number of workgroups: at
+// n = 1,350 with chunks of 256 there were 36, and 32 right-hand sides took
+// 4 x 174 us, now 51.  Halved until every CU has two workgroups, and not below 32, where
+// the partials written and read again would outweigh the matrix.
+int residual_chunk(int nblk, int n, int ngrp)
+{
+  int chunk = RES_CHUNK;
+  while (chunk > 32 && (int64_t)nblk * ((n + chunk - 1) / chunk) * ngrp < 512) chunk /= 2;
+  return chunk;
+}
+
 __global__ __launch_bounds__(256) void k_residual_part(const z2 *__restrict__ M, int64_t ldm, int n,
-                                                       const z2 *__restrict__ X, int64_t ldx, int nrhs, z2 *P)
+                                                       const z2 *__restrict__ X, int64_t ldx, int nrhs, int chunk,
+                                                       z2 *P)
 {
   __shared__ z2 xs[RES_MAXRHS][RES_CHUNK];
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const int c0 = blockIdx.y * RES_CHUNK;
-  const int nc = min(RES_CHUNK, n - c0);
-  for (int idx = threadIdx.x; idx < nrhs * RES_CHUNK; idx += blockDim.x) {
-    const int j = idx / RES_CHUNK, c = idx % RES_CHUNK;
-    xs[j][c] = c < nc ? X[(size_t)j * ldx + c0 + c] : z2{0, 0};
-  }
+  const int c0 = blockIdx.y * chunk;
+  const int nc = min(chunk, n - c0);
+  const int j0 = blockIdx.z * RES_MAXRHS, nj = min(RES_MAXRHS, nrhs - j0);
+  X += (size_t)j0 * ldx;
+  for (int j = 0; j < nj; j++)
+    for (int c = threadIdx.x; c < nc; c += blockDim.x) xs[j][c] = X[(size_t)j * ldx + c0 + c];
   __syncthreads();
   if (r >= n) return;
   double ar[RES_MAXRHS], ai[RES_MAXRHS];
@@ -77,14 +94,14 @@ __global__ __launch_bounds__(256) void k_residual_part(const z2 *__restrict__ M,
     const z2 m = col[(size_t)c * ldm];
 #pragma unroll
     for (int j = 0; j < RES_MAXRHS; j++) {
-      if (j < nrhs) {
+      if (j < nj) {
         const z2 x = xs[j][c];
         ar[j] += m.re * x.re - m.im * x.im;
         ai[j] += m.re * x.im + m.im * x.re;
       }
     }
   }
-  for (int j = 0; j < nrhs; j++) P[((size_t)blockIdx.y * nrhs + j) * n + r] = {ar[j], ai[j]};
+  for (int j = 0; j < nj; j++) P[((size_t)blockIdx.y * nrhs + j0 + j) * n + r] = {ar[j], ai[j]};
 }
 
 // R(:, j) = B(:, j) - sum_chunks P ; partial norms of R and B per block
@@ -163,11 +180,12 @@ extern "C" int bfa_solve_refine(const void *d_M64, int64_t ldm, const void *d_LU
     return fail(BFA_ERR_ARG, "bfa_solve_refine: bad argument");
   hipStream_t st = (hipStream_t)stream;
   if (maxit <= 0) maxit = 10;
-  const int nchunk = (n + RES_CHUNK - 1) / RES_CHUNK;
-  const int nblk = (n + 255) / 256;
+  const int nblk = (n + 255) / 256, nres = std::min(nrhs, RES_BATCH);
+  const int chunk = residual_chunk(nblk, n, (nres + RES_MAXRHS - 1) / RES_MAXRHS);
+  const int nchunk = (n + chunk - 1) / chunk;
   const size_t zsz = (size_t)n * nrhs * sizeof(z2);
   // workspace: B copy (z), X (z), R (z), D (c), partials, norms, solve scratch
-  const size_t part = (size_t)nchunk * std::min(nrhs, RES_MAXRHS) * n * sizeof(z2);
+  const size_t part = (size_t)nchunk * nres * n * sizeof(z2);
   const size_t norms_b = (size_t)2 * nblk * nrhs * sizeof(double);
   const size_t scr = bfa::lu_solve_scratch_bytes(n, nrhs, 8);
   char *w = nullptr;
@@ -197,11 +215,11 @@ extern "C" int bfa_solve_refine(const void *d_M64, int64_t ldm, const void *d_LU
   rc = bfa::lu_solve_prep_c(d_LU32, n, ldlu, d_ipiv, st, scratch);
   for (it = 0; rc == BFA_OK && it <= maxit; it++) {
     if (it > 0) {
-      // r = b - M64 x, in chunks of at most RES_MAXRHS right-hand sides
-      for (int j0 = 0; j0 < nrhs; j0 += RES_MAXRHS) {
-        const int nj = std::min(RES_MAXRHS, nrhs - j0);
-        hipLaunchKernelGGL(k_residual_part, dim3(nblk, nchunk), dim3(256), 0, st, M, ldm, n,
-                           (const z2 *)(X + (size_t)j0 * n), (int64_t)n, nj, P);
+      // r = b - M64 x, RES_BATCH right-hand sides at a time
+      for (int j0 = 0; j0 < nrhs; j0 += RES_BATCH) {
+        const int nj = std::min(RES_BATCH, nrhs - j0);
+        hipLaunchKernelGGL(k_residual_part, dim3(nblk, nchunk, (nj + RES_MAXRHS - 1) / RES_MAXRHS), dim3(256), 0, st,
+                           M, ldm, n, (const z2 *)(X + (size_t)j0 * n), (int64_t)n, nj, chunk, P);
         hipLaunchKernelGGL(k_residual_final, dim3(nblk, nj), dim3(256), 0, st, (const z2 *)P, nchunk, n, nj,
                            (const z2 *)(Bc + (size_t)j0 * n), (int64_t)n, R + (size_t)j0 * n, (int64_t)n,
                            norms + (size_t)2 * nblk * j0);

@@ -60,8 +60,8 @@ struct PanelProb {
 
 
 // Streaming triangular solve of one problem (see k_trsv_stream): the
-// diagonal-block inverses inv [2][n/64][64*64] are built once per
-// factorisation (blk0 also indexes them); each refinement round reads Bin,
+// diagonal-block inverses and their products with the neighbour blocks, inv
+// [4][n/64][64*64], are built once per factorisation (blk0 also indexes them); each refinement round reads Bin,
 // writes the tag-filled Y (forward sweep) and X (backward sweep).
 struct SvProb {
   const void *LU;

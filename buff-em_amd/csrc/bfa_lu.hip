@@ -1458,9 +1458,10 @@ __global__ void k_gather_rows(const cplx<T> *B, int64_t ldb, cplx<T> *X, int64_t
 
 // ---------------------------------------------------------------------------
 // Streaming block substitution.  The diagonal SV_KB x SV_KB blocks of L
-// (unit) and U are inverted once per factorisation (k_trsv_inv); one launch
-// per triangle then solves every row block: a workgroup takes a ticket t
-// (row block t of L, or nblk-1-t of U), accumulates the updates of the
+// (unit) and U are inverted once per factorisation (k_trsv_inv), and the
+// product of each inverse with the block next to it is kept beside it; one
+// launch per triangle then solves every row block: a workgroup takes a ticket
+// t (row block t of L, or nblk-1-t of U), accumulates the updates of the
 // blocks solved before it as they appear, applies its inverted diagonal
 // block and stores its solution.  The output starts filled with a
 // signalling-NaN tag that arithmetic never produces; solved values are
@@ -1471,7 +1472,18 @@ __global__ void k_gather_rows(const cplx<T> *B, int64_t ldb, cplx<T> *X, int64_t
 template <typename T> struct InvShared {
   cplx<T> Ls[SV_KB][SV_KB + 1];
   cplx<T> X[SV_KB][SV_KB + 1];
+  cplx<T> d[SV_KB];
 };
+
+// One diagonal block bi of L or U: its inverse D^-1, and D^-1 A(bi, p) with p
+// the block the sweep solves just before bi (bi - 1 of L, bi + 1 of U).
+// Latency bound: two workgroups per block row and no more, so the chain
+// inside one workgroup is what counts.  Substitution over the 64 columns took
+// 63 barriers (66 us for the complex128 blocks at n = 270); here the four
+// 16 x 16 diagonal blocks are inverted in registers, one wave each, and
+// merged to 32 and 64 by products, with 6 barriers (48 us with the product
+// D^-1 A(bi, p), which the sweeps formed themselves before).  U is held
+// index-reversed so that both triangles are lower ones.
 template <typename T>
 __device__ __forceinline__ void trsv_inv_body(int n, const cplx<T> *__restrict__ A, int64_t lda, cplx<T> *inv, int bi,
                                               bool lower, InvShared<T> &sh)
@@ -1480,30 +1492,129 @@ __device__ __forceinline__ void trsv_inv_body(int n, const cplx<T> *__restrict__
   cplx<T>(&X)[SV_KB][SV_KB + 1] = sh.X;
   const int nblk = (n + SV_KB - 1) / SV_KB;
   const int k0 = bi * SV_KB, kb = min(SV_KB, n - k0);
-  const int tid = threadIdx.x, c = tid % SV_KB, rg = tid / SV_KB;
-  for (int idx = tid; idx < SV_KB * SV_KB; idx += blockDim.x) {
-    const int r = idx % SV_KB, cc = idx / SV_KB;
-    Ls[r][cc] = (r < kb && cc < kb) ? A[(size_t)(k0 + cc) * lda + k0 + r] : cplx<T>{0, 0};
-    X[r][cc] = {(T)(r == cc && r < kb ? 1 : 0), 0};
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int flip = lower ? 0 : SV_KB - 1;
+  for (int idx = tid; idx < SV_KB * SV_KB; idx += 256) {
+    const int r = idx % SV_KB, c = idx / SV_KB;
+    cplx<T> v = {(T)(r == c ? 1 : 0), 0};
+    if (r < kb && c < kb && !(lower && r == c)) v = A[(size_t)(k0 + c) * lda + k0 + r];
+    Ls[r ^ flip][c ^ flip] = v;
   }
   __syncthreads();
-  if (lower) {
-    for (int i = 0; i < kb - 1; i++) {
-      const cplx<T> xi = X[i][c];
-      for (int r = i + 1 + rg; r < kb; r += 4) X[r][c] = c_sub(X[r][c], c_mul(Ls[r][i], xi));
-      __syncthreads();
-    }
-  } else {
-    for (int i = kb - 1; i >= 0; i--) {
-      if (rg == 0) X[i][c] = c_mul(X[i][c], c_inv(Ls[i][i]));
-      __syncthreads();
-      const cplx<T> xi = X[i][c];
-      for (int r = rg; r < i; r += 4) X[r][c] = c_sub(X[r][c], c_mul(Ls[r][i], xi));
-      __syncthreads();
+  if (tid < SV_KB) sh.d[tid] = lower ? cplx<T>{1, 0} : c_inv(Ls[tid][tid]);
+  __syncthreads();
+  if (lane < 16) {
+    const int o = 16 * wv;
+    cplx<T> x[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      cplx<T> v = {(T)(r == lane ? 1 : 0), 0};
+#pragma unroll
+      for (int i = 0; i < r; i++) v = c_sub(v, c_mul(Ls[o + r][o + i], x[i]));
+      x[r] = c_mul(v, sh.d[o + r]);
+      X[o + r][o + lane] = x[r];
     }
   }
+  __syncthreads();
+  // [[A, 0], [C, B]]^-1 = [[A^-1, 0], [-B^-1 (C A^-1), B^-1]]; C A^-1 is put
+  // into the upper triangle of X, which nothing else uses here
+  {
+    const int h = tid >> 7, o = 32 * h, u = tid & 127, r = u & 15, c = 2 * (u >> 4);
+    cplx<T> t0 = {0, 0}, t1 = {0, 0};
+    for (int k = c; k < 16; k++) {
+      const cplx<T> l = Ls[o + 16 + r][o + k];
+      t0 = c_add(t0, c_mul(l, X[o + k][o + c]));
+      if (k > c) t1 = c_add(t1, c_mul(l, X[o + k][o + c + 1]));
+    }
+    X[o + r][o + 16 + c] = t0;
+    X[o + r][o + 16 + c + 1] = t1;
+    __syncthreads();
+    t0 = {0, 0}; t1 = {0, 0};
+    for (int k = 0; k <= r; k++) {
+      const cplx<T> b = X[o + 16 + r][o + 16 + k];
+      t0 = c_sub(t0, c_mul(b, X[o + k][o + 16 + c]));
+      t1 = c_sub(t1, c_mul(b, X[o + k][o + 16 + c + 1]));
+    }
+    X[o + 16 + r][o + c] = t0;
+    X[o + 16 + r][o + c + 1] = t1;
+    __syncthreads();
+    // the temporary of each 32 x 32 block goes back to zero: its inverse is a
+    // factor of the next merge
+    X[o + r][o + 16 + c] = {0, 0};
+    X[o + r][o + 16 + c + 1] = {0, 0};
+    __syncthreads();
+  }
+  {
+    const int r = tid & 15, c = tid >> 4;   // rows r, r + 16, columns c, c + 16
+    cplx<T> t[2][2] = {};
+    for (int k = c; k < 32; k++) {
+      const cplx<T> l0 = Ls[32 + r][k], l1 = Ls[48 + r][k], x0 = X[k][c], x1 = X[k][c + 16];
+      t[0][0] = c_add(t[0][0], c_mul(l0, x0));
+      t[1][0] = c_add(t[1][0], c_mul(l1, x0));
+      t[0][1] = c_add(t[0][1], c_mul(l0, x1));
+      t[1][1] = c_add(t[1][1], c_mul(l1, x1));
+    }
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      X[r + 16 * a][32 + c] = t[a][0];
+      X[r + 16 * a][48 + c] = t[a][1];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 2; a++) { t[a][0] = {0, 0}; t[a][1] = {0, 0}; }
+    for (int k = 0; k <= r + 16; k++) {
+      const cplx<T> l0 = X[32 + r][32 + k], l1 = X[48 + r][32 + k], x0 = X[k][32 + c], x1 = X[k][48 + c];
+      t[0][0] = c_sub(t[0][0], c_mul(l0, x0));
+      t[1][0] = c_sub(t[1][0], c_mul(l1, x0));
+      t[0][1] = c_sub(t[0][1], c_mul(l0, x1));
+      t[1][1] = c_sub(t[1][1], c_mul(l1, x1));
+    }
+    // X[32 + r][32 + k] is zero for k > r: the strict upper triangle of a
+    // merged block was cleared
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      X[32 + r + 16 * a][c] = t[a][0];
+      X[32 + r + 16 * a][c + 16] = t[a][1];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      X[r + 16 * a][32 + c] = {0, 0};
+      X[r + 16 * a][48 + c] = {0, 0};
+    }
+  }
+  // the neighbour block, in the order of X
+  const int kp = lower ? bi - 1 : bi + 1;
+  const bool has = kp >= 0 && kp < nblk;
+  const int cbp = has ? min(SV_KB, n - kp * SV_KB) : 0;
+  if (has)
+    for (int idx = tid; idx < SV_KB * SV_KB; idx += 256) {
+      const int r = idx % SV_KB, c = idx / SV_KB;
+      Ls[r ^ flip][c] = (r < kb && c < cbp) ? A[(size_t)(kp * SV_KB + c) * lda + k0 + r] : cplx<T>{0, 0};
+    }
+  __syncthreads();
   cplx<T> *o = inv + ((size_t)(lower ? 0 : nblk) + bi) * SV_KB * SV_KB;
-  for (int idx = tid; idx < SV_KB * SV_KB; idx += blockDim.x) o[idx] = X[idx % SV_KB][idx / SV_KB];
+  for (int idx = tid; idx < SV_KB * SV_KB; idx += 256) {
+    const int r = idx % SV_KB, c = idx / SV_KB;
+    o[idx] = (r < kb && c < kb) ? X[r ^ flip][c ^ flip] : cplx<T>{0, 0};
+  }
+  if (!has) return;
+  o += (size_t)2 * nblk * SV_KB * SV_KB;
+  const int ty = tid & 15, tx = tid >> 4;   // rows ty + 16 a, columns tx + 16 b
+  cplx<T> m[4][4] = {};
+  for (int k = 0; k < SV_KB; k++) {
+    cplx<T> xa[4], lb[4];
+#pragma unroll
+    for (int a = 0; a < 4; a++) { xa[a] = X[ty + 16 * a][k]; lb[a] = Ls[k][tx + 16 * a]; }
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+      for (int b = 0; b < 4; b++) m[a][b] = c_add(m[a][b], c_mul(xa[a], lb[b]));
+  }
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+#pragma unroll
+    for (int a = 0; a < 4; a++) o[(size_t)(tx + 16 * b) * SV_KB + ((ty + 16 * a) ^ flip)] = m[a][b];
 }
 
 template <typename T>
@@ -1568,192 +1679,169 @@ __global__ void k_sv_reset(cplx<T> *Y, cplx<T> *X, size_t count, unsigned *ticke
   if (i < (size_t)nt) tickets[i] = 0u;
 }
 
+// The waves of a streaming solve: each takes SV_WC of a block's columns, and
+// polls exactly the values it multiplies: column q of right-hand side j is
+// lane q + SV_WC j, so one load per lane covers all of them and they reach
+// the products by readlane, with no LDS and no barrier.
+#define SV_THREADS 512
+#define SV_WAVES (SV_THREADS / 64)
+#define SV_WC (SV_KB / SV_WAVES)
+static_assert(SV_WC * SV_RHS == 64, "one value per lane");
+
 template <typename T> struct StreamShared {
-  cplx<T> xs[SV_RHS][SV_KB];
-  cplx<T> part[4][SV_RHS][SV_KB];
+  cplx<T> part[SV_WAVES][SV_RHS][SV_KB + SV_WC];   // the padding spreads the right-hand sides over the banks
   int ticket;
 };
+
+__device__ __forceinline__ float sv_lane(float v, int l)
+{
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), l));
+}
+__device__ __forceinline__ double sv_lane(double v, int l)
+{
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// acc(:, j) += s * (this wave's columns l) * x(:, j), x one value per lane
+template <typename T>
+__device__ __forceinline__ void sv_product(T (&ar)[SV_RHS], T (&ai)[SV_RHS], const cplx<T> (&l)[SV_WC], cplx<T> x,
+                                           int nrhs)
+{
+#pragma unroll
+  for (int j = 0; j < SV_RHS; j++) {
+    if (j < nrhs) {
+#pragma unroll
+      for (int q = 0; q < SV_WC; q++) {
+        const T xr = sv_lane(x.re, q + SV_WC * j), xi = sv_lane(x.im, q + SV_WC * j);
+        ar[j] += l[q].re * xr - l[q].im * xi;
+        ai[j] += l[q].re * xi + l[q].im * xr;
+      }
+    }
+  }
+}
+
+// wait until the wave's values of one block have landed (bounded: see flag)
+template <typename T>
+__device__ __forceinline__ cplx<T> sv_poll(const cplx<T> *p, bool act, unsigned *flag)
+{
+  cplx<T> v = {0, 0};
+  if (act) {
+    unsigned spins = 0;
+    while (!sv_load(p, v))
+      if (++spins > SPIN_LIMIT) { atomicOr(flag, 1u); break; }
+  }
+  return v;
+}
 
 // Bin: right-hand sides (n x nrhs, read-only here); Xo: tag-filled output.
 // ticket: this sweep's counter; flag: set when a wait gives up.
 // x_i = D_i^-1 (b_i - sum over k != p of L_ik x_k) - (D_i^-1 L_ip) x_p, p the
-// block solved just before i: M = D_i^-1 L_ip is formed while the chain is
-// still upstream, everything but the M x_p term is finished before x_p
-// lands, and the step that waits on x_p is one 64 x 64 product between two
-// workgroup barriers.
+// block solved just before i, the product D_i^-1 L_ip from k_trsv_inv:
+// everything but that term is finished before x_p lands.
+// Bound by the chain of n / 64 blocks: a link is the poll of x_p, 8 columns a
+// wave of one 64 x 64 product, one sum over the waves in LDS and the store.
+// With 4 waves that shared x through LDS (two barriers and a poll by one wave
+// a block, the product D_i^-1 L_ip formed in the sweep) a link took 6-7 us
+// with one right-hand side and 17 with eight; now 2.3 and 4.6 (complex64,
+// n = 19,440: 1.9 -> 0.69 ms a sweep, 1.5 GB of the triangle at 2.2 TB/s).
 template <typename T, bool LOWER>
 __device__ __forceinline__ void trsv_stream_body(int n, int nrhs, const cplx<T> *__restrict__ A, int64_t lda,
                                                  const cplx<T> *__restrict__ inv, const cplx<T> *Bin, cplx<T> *Xo,
                                                  int64_t ldx, unsigned *ticket, unsigned *flag, StreamShared<T> &sh)
 {
   const int nblk = (n + SV_KB - 1) / SV_KB;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (tid == 0) sh.ticket = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  const int t = sh.ticket;
+  const int t = __builtin_amdgcn_readfirstlane(sh.ticket);
   const int bi = LOWER ? t : nblk - 1 - t;
   const int r0 = bi * SV_KB, kb = min(SV_KB, n - r0);
   const int r = r0 + lane;
-  // this wave's columns of the inverted diagonal block, loaded up front
-  const cplx<T> *Di = inv + ((size_t)(LOWER ? 0 : nblk) + bi) * SV_KB * SV_KB;
-  cplx<T> dcol[SV_KB / 4];
+  const int w0 = wv * SV_WC;                       // the wave's first column of every block
+  const int xc = w0 + lane % SV_WC, xj = lane / SV_WC;   // the lane's value of a block
+  const size_t xo = (size_t)xj * ldx + xc;
+  const cplx<T> bv = (xj < nrhs && xc < kb) ? Bin[(size_t)r0 + xo] : cplx<T>{0, 0};
+  // this wave's columns of the inverted diagonal block and of D^-1 L_ip
+  const cplx<T> *Di = inv + ((size_t)(LOWER ? 0 : nblk) + bi) * SV_KB * SV_KB + (size_t)w0 * SV_KB + lane;
+  const cplx<T> *Mi = Di + (size_t)2 * nblk * SV_KB * SV_KB;
+  cplx<T> dcol[SV_WC], mcol[SV_WC];
 #pragma unroll
-  for (int q = 0; q < SV_KB / 4; q++) dcol[q] = Di[(size_t)(wv + 4 * q) * SV_KB + lane];
-  // M = D^-1 L_ip, this thread's row (lane) and the wave's columns: row tt of
-  // block (i, p) is held by lane tt of the wave, passed along by shuffles
-  const int kp = t > 0 ? (LOWER ? t - 1 : nblk - t) : 0;
-  const int cp0 = kp * SV_KB, cbp = t > 0 ? min(SV_KB, n - cp0) : 0;
-  cplx<T> mcol[SV_KB / 4];
-#pragma unroll
-  for (int q = 0; q < SV_KB / 4; q++) mcol[q] = {0, 0};
-  if (t > 0) {
-    cplx<T> lp[SV_KB / 4];
-#pragma unroll
-    for (int q = 0; q < SV_KB / 4; q++) {
-      const int c = wv + 4 * q;
-      lp[q] = (lane < kb && c < cbp) ? A[(size_t)(cp0 + c) * lda + r] : cplx<T>{0, 0};
-    }
-    for (int tt = 0; tt < SV_KB; tt++) {
-      const cplx<T> d = Di[(size_t)tt * SV_KB + lane];      // D^-1 (lane, tt)
-#pragma unroll
-      for (int q = 0; q < SV_KB / 4; q++) {
-        const T pr = __shfl(lp[q].re, tt, 64), pi = __shfl(lp[q].im, tt, 64);
-        mcol[q].re += d.re * pr - d.im * pi;
-        mcol[q].im += d.re * pi + d.im * pr;
-      }
-    }
+  for (int q = 0; q < SV_WC; q++) {
+    dcol[q] = Di[(size_t)q * SV_KB];
+    mcol[q] = t > 0 ? Mi[(size_t)q * SV_KB] : cplx<T>{0, 0};
   }
   T ar[SV_RHS], ai[SV_RHS];
 #pragma unroll
   for (int j = 0; j < SV_RHS; j++) { ar[j] = 0; ai[j] = 0; }
-  for (int s = 0; s < t - 1; s++) {
+  // this wave's columns of block (bi, k) of step s, two steps ahead of their
+  // use (and issued after the poll of the step between: a wave's loads return
+  // in order, so a poll waits for every load before it)
+  auto tile = [&](cplx<T> (&l)[SV_WC], int s) __attribute__((always_inline)) {
     const int k = LOWER ? s : nblk - 1 - s;
-    const int c0 = k * SV_KB, cb = min(SV_KB, n - c0);
-    // this wave's columns of block (bi, k), loaded before waiting on x_k
-    cplx<T> l[SV_KB / 4];
+    const int c0 = k * SV_KB + w0, cb = n - c0;
 #pragma unroll
-    for (int q = 0; q < SV_KB / 4; q++) {
-      const int c = wv + 4 * q;
-      l[q] = (lane < kb && c < cb) ? A[(size_t)(c0 + c) * lda + r] : cplx<T>{0, 0};
-    }
-    // wave 0 polls x_k until every value has landed
-    if (wv == 0) {
-      unsigned spins = 0;
-      for (int idx = lane; idx < cb * nrhs; idx += 64) {
-        const int c = idx % cb, j = idx / cb;
-        cplx<T> v;
-        while (!sv_load(&Xo[(size_t)j * ldx + c0 + c], v)) {
-          if (++spins > SPIN_LIMIT) { atomicOr(flag, 1u); break; }
-        }
-        sh.xs[j][c] = v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < SV_KB / 4; q++) {
-      const int c = wv + 4 * q;
-#pragma unroll
-      for (int j = 0; j < SV_RHS; j++) {
-        if (j < nrhs) {
-          const cplx<T> x = sh.xs[j][c < cb ? c : 0];
-          ar[j] += l[q].re * x.re - l[q].im * x.im;
-          ai[j] += l[q].re * x.im + l[q].im * x.re;
-        }
-      }
-    }
-    __syncthreads();
+    for (int q = 0; q < SV_WC; q++)
+      l[q] = (lane < kb && q < cb) ? A[(size_t)(c0 + q) * lda + r] : cplx<T>{0, 0};
+  };
+  auto value = [&](int s) __attribute__((always_inline)) {
+    const int c0 = (LOWER ? s : nblk - 1 - s) * SV_KB;
+    return sv_poll(Xo + c0 + xo, xj < nrhs && c0 + xc < n, flag);
+  };
+  cplx<T> l0[SV_WC], l1[SV_WC];
+  if (t > 1) tile(l0, 0);
+  if (t > 2) tile(l1, 1);
+  int s = 0;
+  for (; s + 1 < t - 1; s += 2) {
+    cplx<T> x = value(s);
+    sv_product<T>(ar, ai, l0, x, nrhs);
+    if (s + 2 < t - 1) tile(l0, s + 2);
+    x = value(s + 1);
+    sv_product<T>(ar, ai, l1, x, nrhs);
+    if (s + 3 < t - 1) tile(l1, s + 3);
   }
+  if (s < t - 1) sv_product<T>(ar, ai, l0, value(s), nrhs);
   for (int j = 0; j < nrhs; j++) sh.part[wv][j][lane] = {ar[j], ai[j]};
   __syncthreads();
-  // raw right-hand side of this block without x_p's term: b - sum of updates
-  if (wv == 0) {
-    for (int j = 0; j < nrhs; j++) {
-      cplx<T> v = {0, 0};
-      if (lane < kb) {
-        const cplx<T> b = Bin[(size_t)j * ldx + r];
-        v.re = b.re - (sh.part[0][j][lane].re + sh.part[1][j][lane].re + sh.part[2][j][lane].re + sh.part[3][j][lane].re);
-        v.im = b.im - (sh.part[0][j][lane].im + sh.part[1][j][lane].im + sh.part[2][j][lane].im + sh.part[3][j][lane].im);
-      }
-      sh.xs[j][lane] = v;
-    }
+  // b - sum of updates without x_p's term, each wave the values of its columns
+  cplx<T> x = bv;
+  if (xj < nrhs) {
+#pragma unroll
+    for (int w = 0; w < SV_WAVES; w++) x = c_sub(x, sh.part[w][xj][xc]);
   }
   __syncthreads();
-  // z = inv(D) * raw, D the diagonal block
 #pragma unroll
   for (int j = 0; j < SV_RHS; j++) { ar[j] = 0; ai[j] = 0; }
-#pragma unroll
-  for (int q = 0; q < SV_KB / 4; q++) {
-    const int c = wv + 4 * q;
-    const cplx<T> d = dcol[q];
-#pragma unroll
-    for (int j = 0; j < SV_RHS; j++) {
-      if (j < nrhs) {
-        const cplx<T> x = sh.xs[j][c];
-        ar[j] += d.re * x.re - d.im * x.im;
-        ai[j] += d.re * x.im + d.im * x.re;
-      }
-    }
+  sv_product<T>(ar, ai, dcol, x, nrhs);
+  if (t > 0) {
+    x = value(t - 1);
+    x = {-x.re, -x.im};
+    sv_product<T>(ar, ai, mcol, x, nrhs);
   }
   for (int j = 0; j < nrhs; j++) sh.part[wv][j][lane] = {ar[j], ai[j]};
   __syncthreads();
-  T zr[SV_RHS], zi[SV_RHS];
+  if (wv < nrhs && lane < kb) {
+    cplx<T> v = sh.part[0][wv][lane];
 #pragma unroll
-  for (int j = 0; j < SV_RHS; j++) {
-    zr[j] = zi[j] = 0;
-    if (wv == 0 && j < nrhs) {
-      zr[j] = sh.part[0][j][lane].re + sh.part[1][j][lane].re + sh.part[2][j][lane].re + sh.part[3][j][lane].re;
-      zi[j] = sh.part[0][j][lane].im + sh.part[1][j][lane].im + sh.part[2][j][lane].im + sh.part[3][j][lane].im;
-    }
-  }
-  if (t > 0) {
-    // wave 0 polls x_p (xs is free: every wave read it before the last barrier)
-    if (wv == 0) {
-      unsigned spins = 0;
-      for (int idx = lane; idx < cbp * nrhs; idx += 64) {
-        const int c = idx % cbp, j = idx / cbp;
-        cplx<T> v;
-        while (!sv_load(&Xo[(size_t)j * ldx + cp0 + c], v)) {
-          if (++spins > SPIN_LIMIT) { atomicOr(flag, 1u); break; }
-        }
-        sh.xs[j][c] = v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < SV_RHS; j++) { ar[j] = 0; ai[j] = 0; }
-#pragma unroll
-    for (int q = 0; q < SV_KB / 4; q++) {
-      const int c = wv + 4 * q;
-#pragma unroll
-      for (int j = 0; j < SV_RHS; j++) {
-        if (j < nrhs) {
-          const cplx<T> x = sh.xs[j][c < cbp ? c : 0];
-          ar[j] += mcol[q].re * x.re - mcol[q].im * x.im;
-          ai[j] += mcol[q].re * x.im + mcol[q].im * x.re;
-        }
-      }
-    }
-    for (int j = 0; j < nrhs; j++) sh.part[wv][j][lane] = {ar[j], ai[j]};
-    __syncthreads();
-    if (wv == 0 && lane < kb) {
-      for (int j = 0; j < nrhs; j++) {
-        const T mr = sh.part[0][j][lane].re + sh.part[1][j][lane].re + sh.part[2][j][lane].re + sh.part[3][j][lane].re;
-        const T mi = sh.part[0][j][lane].im + sh.part[1][j][lane].im + sh.part[2][j][lane].im + sh.part[3][j][lane].im;
-        sv_store(&Xo[(size_t)j * ldx + r], cplx<T>{zr[j] - mr, zi[j] - mi});
-      }
-    }
-  } else if (wv == 0 && lane < kb) {
-    for (int j = 0; j < nrhs; j++) sv_store(&Xo[(size_t)j * ldx + r], cplx<T>{zr[j], zi[j]});
+    for (int w = 1; w < SV_WAVES; w++) v = c_add(v, sh.part[w][wv][lane]);
+    sv_store(&Xo[(size_t)wv * ldx + r], v);
   }
 }
+static_assert(SV_WAVES >= SV_RHS, "one wave stores one right-hand side");
 
+// blockIdx.y: a group of SV_RHS right-hand sides with tickets of its own, so
+// the chains of the groups run side by side
 template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void k_trsv_stream(int n, int nrhs, const cplx<T> *__restrict__ A, int64_t lda,
-                                                     const cplx<T> *__restrict__ inv, const cplx<T> *Bin,
-                                                     cplx<T> *Xo, int64_t ldx, unsigned *ticket, unsigned *flag)
+__global__ __launch_bounds__(SV_THREADS) void k_trsv_stream(int n, int nrhs, const cplx<T> *__restrict__ A,
+                                                            int64_t lda, const cplx<T> *__restrict__ inv,
+                                                            const cplx<T> *Bin, cplx<T> *Xo, int64_t ldx,
+                                                            unsigned *tickets, unsigned *flag)
 {
   __shared__ StreamShared<T> sh;
-  trsv_stream_body<T, LOWER>(n, nrhs, A, lda, inv, Bin, Xo, ldx, ticket, flag, sh);
+  const int c = blockIdx.y, j0 = c * SV_RHS;
+  const size_t o = (size_t)j0 * ldx;
+  trsv_stream_body<T, LOWER>(n, min(SV_RHS, nrhs - j0), A, lda, inv, Bin + o, Xo + o, ldx,
+                             tickets + 2 * c + (LOWER ? 0 : 1), flag, sh);
 }
 
 // grouped forms over the problems of a batch (complex64)
@@ -1766,7 +1854,7 @@ __global__ __launch_bounds__(256) void kg_sv_inv(const SvProb *__restrict__ d, i
 }
 
 template <bool LOWER>
-__global__ __launch_bounds__(256) void kg_sv_stream(const SvProb *__restrict__ d, int np)
+__global__ __launch_bounds__(SV_THREADS) void kg_sv_stream(const SvProb *__restrict__ d, int np)
 {
   __shared__ StreamShared<float> sh;
   const SvProb q = d[find_prob(d, np, blockIdx.x)];
@@ -1776,14 +1864,14 @@ __global__ __launch_bounds__(256) void kg_sv_stream(const SvProb *__restrict__ d
                                  q.tick + (LOWER ? 0 : 1), (unsigned *)q.flag, sh);
 }
 
-// scratch: [perm n ints][flag 256 B][inverted diagonal blocks]
+// scratch: [perm n ints][flag 256 B][inverted diagonal blocks, their products]
 //          [P b, Y, X: n x nrhs each][tickets]
 static size_t sv_align(size_t x) { return (x + 255) / 256 * 256; }
 static size_t sv_inv_off(int n) { return sv_align((size_t)n * 4) + 256; }
 static size_t sv_x_off(int n, size_t elem)
 {
   const size_t nblk = (size_t)(n + SV_KB - 1) / SV_KB;
-  return sv_inv_off(n) + sv_align(2 * nblk * SV_KB * SV_KB * elem);
+  return sv_inv_off(n) + sv_align(4 * nblk * SV_KB * SV_KB * elem);
 }
 static int sv_nticket(int nrhs) { return 2 * ((nrhs + SV_RHS - 1) / SV_RHS); }
 
@@ -1868,14 +1956,11 @@ int lu_solve_apply(const cplx<T> *A, int n, int64_t lda, cplx<T> *B, int nrhs, i
   hipLaunchKernelGGL(k_sv_reset<T>, dim3((unsigned)((std::max(count, (size_t)nt) + 255) / 256)), dim3(256), 0, st, Y,
                      X, count, tickets, nt);
   const int nblk = (n + SV_KB - 1) / SV_KB;
-  for (int j0 = 0, c = 0; j0 < nrhs; j0 += SV_RHS, c++) {
-    const int nj = std::min(SV_RHS, nrhs - j0);
-    const size_t o = (size_t)j0 * n;
-    hipLaunchKernelGGL((k_trsv_stream<T, true>), dim3(nblk), dim3(256), 0, st, n, nj, A, lda, inv,
-                       (const cplx<T> *)(Pb + o), Y + o, (int64_t)n, tickets + 2 * c, flag);
-    hipLaunchKernelGGL((k_trsv_stream<T, false>), dim3(nblk), dim3(256), 0, st, n, nj, A, lda, inv,
-                       (const cplx<T> *)(Y + o), X + o, (int64_t)n, tickets + 2 * c + 1, flag);
-  }
+  const dim3 grid(nblk, (nrhs + SV_RHS - 1) / SV_RHS);
+  hipLaunchKernelGGL((k_trsv_stream<T, true>), grid, dim3(SV_THREADS), 0, st, n, nrhs, A, lda, inv,
+                     (const cplx<T> *)Pb, Y, (int64_t)n, tickets, flag);
+  hipLaunchKernelGGL((k_trsv_stream<T, false>), grid, dim3(SV_THREADS), 0, st, n, nrhs, A, lda, inv,
+                     (const cplx<T> *)Y, X, (int64_t)n, tickets, flag);
   HIPCHECK(hipMemcpy2DAsync(B, ldb * sizeof(cplx<T>), X, n * sizeof(cplx<T>), n * sizeof(cplx<T>), nrhs,
                             hipMemcpyDeviceToDevice, st));
   HIPCHECK(hipGetLastError());
@@ -1987,8 +2072,8 @@ void launch_sv_inv_g(const SvProb *d, int np, int nblk, hipStream_t st)
 void launch_sv_stream_g(bool lower, const SvProb *d, int np, int nblk, hipStream_t st)
 {
   if (np <= 0 || nblk <= 0) return;
-  if (lower) hipLaunchKernelGGL(kg_sv_stream<true>, dim3(nblk), dim3(256), 0, st, d, np);
-  else hipLaunchKernelGGL(kg_sv_stream<false>, dim3(nblk), dim3(256), 0, st, d, np);
+  if (lower) hipLaunchKernelGGL(kg_sv_stream<true>, dim3(nblk), dim3(SV_THREADS), 0, st, d, np);
+  else hipLaunchKernelGGL(kg_sv_stream<false>, dim3(nblk), dim3(SV_THREADS), 0, st, d, np);
 }
 int panel_sync_words() { return PB_WORDS; }
 unsigned long long sv_tag_c64() { return (unsigned long long)SvTag<float>::bits * 0x100000001ull; }

@@ -1,13 +1,13 @@
 // bfa_noalloc.hip -- an LU solve that allocates no device memory.
 //
 // bfa_lu_solve_z allocates its scratch (row permutation, timeout flag,
-// inverted 64 x 64 diagonal blocks of L and U, the permuted right-hand
-// sides, the forward and backward solutions and the streaming solves'
-// tickets) with hipMalloc on every call.  Callers that cannot allocate --
+// inverted 64 x 64 diagonal blocks of L and U and their products with the
+// neighbour blocks, the permuted right-hand sides, the forward and backward
+// solutions and the streaming solves' tickets) with hipMalloc on every call.  Callers that cannot allocate --
 // code under HIP graph capture, tight serving loops, harnesses that forbid
 // it -- use bfa_lu_solve_z_noalloc instead: the same kernels, with the
 // scratch in one statically sized device array per GPU, sized for
-// n <= BFA_NOALLOC_MAX_N and nrhs <= BFA_NOALLOC_MAX_NRHS (47.6 MiB, held by
+// n <= BFA_NOALLOC_MAX_N and nrhs <= BFA_NOALLOC_MAX_NRHS (87.6 MiB, held by
 // every device the library runs on until the process ends).
 //
 // Every call on a device uses that device's one array, so calls that
@@ -25,10 +25,10 @@ namespace {
 constexpr size_t al256(size_t x) { return (x + 255) / 256 * 256; }
 
 // the layout of lu_solve's scratch for the streaming form (nrhs < 64):
-// [perm n ints][flag 256 B][2 x nblk inverted 64 x 64 blocks][P b, Y, X][tickets]
+// [perm n ints][flag 256 B][4 x nblk 64 x 64 blocks: inverses, products][P b, Y, X][tickets]
 constexpr size_t noalloc_bytes(size_t n, size_t nrhs)
 {
-  return al256(n * 4) + 256 + al256(2 * ((n + 63) / 64) * 64 * 64 * 16) + 3 * al256(n * nrhs * 16) +
+  return al256(n * 4) + 256 + al256(4 * ((n + 63) / 64) * 64 * 64 * 16) + 3 * al256(n * nrhs * 16) +
          al256(2 * ((nrhs + 7) / 8) * 4);
 }
 

@@ -206,7 +206,7 @@ int  bfa_lu_solve_z(const void *d_A, int n, int64_t lda, const int *d_ipiv,
  * for callers that cannot call hipMalloc -- code under HIP graph capture,
  * tight serving loops, harnesses that forbid allocation.  Same kernels and
  * results as bfa_lu_solve_z; its scratch is one static device array per GPU
- * (47.6 MiB, kept until the process ends), so n <= BFA_NOALLOC_MAX_N and
+ * (87.6 MiB, kept until the process ends), so n <= BFA_NOALLOC_MAX_N and
  * nrhs <= BFA_NOALLOC_MAX_NRHS (larger sizes return BFA_ERR_ARG), and calls
  * that overlap on one GPU race on that array.  Synchronous like
  * bfa_lu_solve_z.                                                          */
