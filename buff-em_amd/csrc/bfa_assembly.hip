@@ -195,14 +195,30 @@ extern "C" int bfa_geometry_upload(bfa_geometry *g, void *stream)
 
 // ===========================================================================
 // Cold step 1: Taylor-Duffy moments.  One workgroup per tetrahedron pair.
-// Structure identical to the oracle's orc_td_moments: per base simplex the
-// displacement L, and the radial coefficients X1, Y1 are affine in sigma;
-// the radial and remaining-variable integrals are closed-form (Beta
-// integrals, simplex covariance).
+// Per base simplex the displacement L and the radial coefficients X1 and
+// Y1 = X1 + L (the columns of Mx and My that multiply the remaining variables
+// belong to the common vertices) are affine in sigma; the radial and
+// remaining-variable integrals are closed-form (Beta integrals, simplex
+// covariance).  Bound by FP64 instructions.  The collapsed coordinates are
+// t_d = g_0 g_1 ... g_d, so along the last one L = LA + g LB and
+// X1 = XA + g XB: a thread takes one line of n nodes and sums f, f g and
+// f g^2 for f = w/r and w r (w alone gives constants), about 25 instructions a
+// node, and turns them into the 24 moments once a line (~150).  Point by
+// point, with the barycentric coordinates read from a table, a node took ~115
+// and the pairs of a 3,072-tetrahedron ball (order 12) 20.5 ms; now 7.6 ms,
+// what the FP64 instructions of 7.7e9 nodes take to issue.
 // ===========================================================================
-struct TDPoints {
-  const double *lam[3];   // case c: [(D+1) * npts], layout lam0[npts],...,lamD-1[npts], wt[npts]
-  int npts[3];
+#define TD_MAXORDER 32
+struct TDNodes {          // Gauss nodes and weights on [0, 1] for 4, 3, 2 common vertices
+  double x[3][TD_MAXORDER], w[3][TD_MAXORDER];
+  int n[3];
+};
+struct TDShared {
+  double E[20][5][6];     // per simplex: L, X1 at vertex 0, then the edges between successive vertices
+  double det[20];
+  double red[4 * 24];
+  double x[TD_MAXORDER], w[TD_MAXORDER], wx[TD_MAXORDER], wxx[TD_MAXORDER], ww[3];
+  double Mx[3][3], My[3][3], cov[3][3], tbar[3], tot[24];
 };
 
 template <int NCV> struct TDCase;
@@ -247,11 +263,13 @@ __device__ __forceinline__ double wave_sum(double v)
 }
 
 template <int NCV>
-__device__ void td_pair(const double *VA, const double *VB, const double *cA, const double *cB,
-                        const double *lam, int npts, double *out, double *red)
+__device__ void td_pair(const double *VA, const double *VB, const double *cA, const double *cB, const TDNodes &td,
+                        int ic, double *out, TDShared &sh)
 {
   using C = TDCase<NCV>;
-  constexpr int D = C::D, M = C::M;
+  constexpr int D = C::D, M = C::M, K = D - 1;
+  static_assert(C::NSIMP <= 20 && D <= 5, "TDShared");
+  const int n = td.n[ic];
   const int tid = threadIdx.x;
   double Mx[3][3], My[3][3];
   for (int d = 0; d < 3; d++) {
@@ -301,74 +319,137 @@ __device__ void td_pair(const double *VA, const double *VB, const double *cA, co
       for (int a = 0; a < M; a++)
         for (int b = 0; b < M; b++) cov[a][b] += tw[i] * (tau[i][a] - tbar[a]) * (tau[i][b] - tbar[b]) / vol;
   }
+  if (tid < n) {
+    const double x = td.x[ic][tid], w = td.w[ic][tid];
+    sh.x[tid] = x;
+    sh.w[tid] = w;
+    sh.wx[tid] = w * x;
+    sh.wxx[tid] = w * x * x;
+  }
+  if (tid < C::NSIMP) sh.det[tid] = C::det(tid);
+  if (tid == 0) {   // for the last step: not held in registers over the loop
+    for (int d = 0; d < 3; d++) {
+      sh.tbar[d] = tbar[d];
+      for (int c = 0; c < 3; c++) { sh.Mx[d][c] = Mx[d][c]; sh.My[d][c] = My[d][c]; sh.cov[d][c] = cov[d][c]; }
+    }
+  }
   // rem -> physical maps: the first M columns of Mx / My
-  double acc[3][8];
-  for (int p = 0; p < 3; p++)
-    for (int q = 0; q < 8; q++) acc[p][q] = 0.0;
-  const double *wt = lam + (size_t)D * npts;
-  for (int is = 0; is < C::NSIMP; is++) {
-    const double *sv = C::simp(is);
-    const double *O = C::off(is);
-    const double sdet = C::det(is);
-    double Lv[D][3], X1v[D][3], Y1v[D][3];
-#pragma unroll
-    for (int q = 0; q < D; q++) {
-      const double *s = sv + q * D;
+  if (tid < C::NSIMP * D) {
+    const int is = tid / D, q = tid % D;
+    const double *sv = C::simp(is), *O = C::off(is);
+    double v[2][6];
+    for (int e = 0; e < 2; e++) {
+      const double *s = sv + (q > 0 ? q - 1 + e : 0) * D;
       double rem[3], xs[3], es[3];
       for (int a = 0; a < M; a++) {
-        double v = 0.0;
-        for (int d = 0; d < D; d++) v += O[a * D + d] * s[d];
-        rem[a] = v - tbar[a];
+        double o = 0.0;
+        for (int d = 0; d < D; d++) o += O[a * D + d] * s[d];
+        rem[a] = o - tbar[a];
       }
       td_split<NCV>(s, xs, es);
       for (int d = 0; d < 3; d++) {
-        double l = 0, x1 = 0, y1 = 0;
+        double l = 0, x1 = 0;
         for (int c = 0; c < 3; c++) {
           l += My[d][c] * es[c] - Mx[d][c] * xs[c];
           x1 += Mx[d][c] * xs[c];
-          y1 += My[d][c] * es[c];
         }
-        for (int a = 0; a < M; a++) { x1 += Mx[d][a] * rem[a]; y1 += My[d][a] * rem[a]; }
-        Lv[q][d] = l; X1v[q][d] = x1; Y1v[q][d] = y1;
+        for (int a = 0; a < M; a++) x1 += Mx[d][a] * rem[a];
+        v[e][d] = l; v[e][3 + d] = x1;
       }
     }
-    for (int ip = tid; ip < npts; ip += blockDim.x) {
-      double L[3] = {0, 0, 0}, X1[3] = {0, 0, 0}, Y1[3] = {0, 0, 0};
+    for (int d = 0; d < 6; d++) sh.E[is][q][d] = q > 0 ? v[1][d] - v[0][d] : v[0][d];
+  }
+  __syncthreads();
+  if (tid < 3) {
+    double c = 0.0;
+    for (int i = 0; i < n; i++) c += tid == 0 ? sh.w[i] : tid == 1 ? sh.wx[i] : sh.wxx[i];
+    sh.ww[tid] = c;
+  }
+  __syncthreads();
+  double acc[3][8];
 #pragma unroll
-      for (int q = 0; q < D; q++) {
-        double l = lam[(size_t)q * npts + ip];
+  for (int p = 0; p < 3; p++)
 #pragma unroll
-        for (int d = 0; d < 3; d++) { L[d] += l * Lv[q][d]; X1[d] += l * X1v[q][d]; Y1[d] += l * Y1v[q][d]; }
+    for (int q = 0; q < 8; q++) acc[p][q] = 0.0;
+  unsigned nl = 1;
+  for (int d = 0; d < K - 1; d++) nl *= n;
+  for (unsigned task = tid; task < C::NSIMP * nl; task += 256) {
+    const unsigned is = task / nl;
+    unsigned ri = task - is * nl;
+    const double *E = &sh.E[is][0][0];
+    double LX[6], LXg[6];
+#pragma unroll
+    for (int d = 0; d < 6; d++) LX[d] = E[d];
+    double W = sh.det[is], t = 1.0;
+#pragma unroll
+    for (int d = 0; d < K - 1; d++) {
+      const unsigned rn = ri / n, id = ri - rn * n;
+      ri = rn;
+      const double v = sh.x[id];
+      t *= v;
+      W *= sh.w[id];
+#pragma unroll
+      for (int e = 0; e < K - 1 - d; e++) W *= v;
+#pragma unroll
+      for (int c = 0; c < 6; c++) LX[c] += t * E[6 * (d + 1) + c];
+    }
+#pragma unroll
+    for (int c = 0; c < 6; c++) LXg[c] = t * E[6 * K + c];
+    double s[3][3] = {};
+#pragma unroll 2
+    for (int i = 0; i < n; i++) {
+      const double gx = sh.x[i], w0 = sh.w[i], w1 = sh.wx[i], w2 = sh.wxx[i];
+      const double L0 = LX[0] + gx * LXg[0], L1 = LX[1] + gx * LXg[1], L2 = LX[2] + gx * LXg[2];
+      const double r2 = L0 * L0 + L1 * L1 + L2 * L2;
+      const double f0 = rsqrt_nr(r2), f2 = f0 * r2;
+      s[0][0] += w0 * f0; s[0][1] += w1 * f0; s[0][2] += w2 * f0;
+      s[2][0] += w0 * f2; s[2][1] += w1 * f2; s[2][2] += w2 * f2;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) s[1][q] = sh.ww[q];
+    const double *XA = LX + 3, *XB = LXg + 3;
+    double YA[3], YB[3], aa = 0, ab = 0, bb = 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      YA[d] = XA[d] + LX[d]; YB[d] = XB[d] + LXg[d];
+      aa += XA[d] * YA[d];
+      ab += XA[d] * YB[d] + XB[d] * YA[d];
+      bb += XB[d] * YB[d];
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      const double m0 = W * s[p][0], m1 = W * s[p][1], m2 = W * s[p][2];
+      acc[p][0] += m0;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        acc[p][1 + d] += m0 * XA[d] + m1 * XB[d];
+        acc[p][4 + d] += m0 * YA[d] + m1 * YB[d];
       }
-      double r = sqrt(L[0] * L[0] + L[1] * L[1] + L[2] * L[2]);
-      double w = sdet * wt[ip];
-      double xy = X1[0] * Y1[0] + X1[1] * Y1[1] + X1[2] * Y1[2];
-      double f[3] = {w / r, w, w * r};
-#pragma unroll
-      for (int p = 0; p < 3; p++) {
-        acc[p][0] += f[p];
-        acc[p][1] += f[p] * X1[0]; acc[p][2] += f[p] * X1[1]; acc[p][3] += f[p] * X1[2];
-        acc[p][4] += f[p] * Y1[0]; acc[p][5] += f[p] * Y1[1]; acc[p][6] += f[p] * Y1[2];
-        acc[p][7] += f[p] * xy;
-      }
+      acc[p][7] += m0 * aa + m1 * ab + m2 * bb;
     }
   }
   // block reduction of the 24 accumulators
+  double *red = sh.red;
   const int lane = tid & 63, wid = tid >> 6, nw = blockDim.x >> 6;
+#pragma unroll
   for (int p = 0; p < 3; p++)
+#pragma unroll
     for (int q = 0; q < 8; q++) {
       double v = wave_sum(acc[p][q]);
       if (lane == 0) red[wid * 24 + p * 8 + q] = v;
     }
   __syncthreads();
-  if (tid == 0) {
-    double tot[3][8];
-    for (int p = 0; p < 3; p++)
-      for (int q = 0; q < 8; q++) {
-        double s = 0.0;
-        for (int w = 0; w < nw; w++) s += red[w * 24 + p * 8 + q];
-        tot[p][q] = s;
-      }
+  if (tid < 24) {
+    double v = 0.0;
+    for (int w = 0; w < nw; w++) v += red[w * 24 + tid];
+    sh.tot[tid] = v;
+  }
+  __syncthreads();
+  if (tid < 3) {   // one kernel power each
+    const int p = tid;
+    const double *tot = sh.tot + 8 * p;
+    const auto &Mx = sh.Mx, &My = sh.My, &cov = sh.cov;
+    const auto &tbar = sh.tbar;
     double detA = Mx[0][0] * (Mx[1][1] * Mx[2][2] - Mx[2][1] * Mx[1][2])
                 - Mx[0][1] * (Mx[1][0] * Mx[2][2] - Mx[2][0] * Mx[1][2])
                 + Mx[0][2] * (Mx[1][0] * Mx[2][1] - Mx[2][0] * Mx[1][1]);
@@ -385,35 +466,35 @@ __device__ void td_pair(const double *VA, const double *VB, const double *cA, co
       for (int b = 0; b < M; b++)
         kappa += cov[a][b] * (Mx[0][a] * My[0][b] + Mx[1][a] * My[1][b] + Mx[2][a] * My[2][b]);
     double s0 = jac * vol;
-    for (int p = 0; p < 3; p++) {
+    {
       double b0 = beta_int(D - 2 + p, M), b1 = beta_int(D - 1 + p, M), b2 = beta_int(D + p, M);
       double bk = beta_int(D - 2 + p, M + 2);
-      double a0 = tot[p][0];
+      double a0 = tot[0];
       out[p * 8] = s0 * b0 * a0;
       for (int d = 0; d < 3; d++) {
-        out[p * 8 + 1 + d] = s0 * (b0 * X0[d] * a0 + b1 * tot[p][1 + d]);
-        out[p * 8 + 4 + d] = s0 * (b0 * Y0[d] * a0 + b1 * tot[p][4 + d]);
+        out[p * 8 + 1 + d] = s0 * (b0 * X0[d] * a0 + b1 * tot[1 + d]);
+        out[p * 8 + 4 + d] = s0 * (b0 * Y0[d] * a0 + b1 * tot[4 + d]);
       }
       double x0y0 = X0[0] * Y0[0] + X0[1] * Y0[1] + X0[2] * Y0[2];
-      double cross = X0[0] * tot[p][4] + X0[1] * tot[p][5] + X0[2] * tot[p][6]
-                   + Y0[0] * tot[p][1] + Y0[1] * tot[p][2] + Y0[2] * tot[p][3];
-      out[p * 8 + 7] = s0 * (b0 * x0y0 * a0 + b1 * cross + b2 * tot[p][7] + bk * kappa * a0);
+      double cross = X0[0] * tot[4] + X0[1] * tot[5] + X0[2] * tot[6]
+                   + Y0[0] * tot[1] + Y0[1] * tot[2] + Y0[2] * tot[3];
+      out[p * 8 + 7] = s0 * (b0 * x0y0 * a0 + b1 * cross + b2 * tot[7] + bk * kappa * a0);
     }
   }
 }
 
 __global__ __launch_bounds__(256) void k_td_moments(const int *pairs, const double *verts,
-                                                    const double *tetCen, TDPoints tp, double *mom)
+                                                    const double *tetCen, TDNodes td, double *mom)
 {
-  __shared__ double red[4 * 24];
+  __shared__ TDShared sh;
   const int p = blockIdx.x;
   const int tA = pairs[4 * p], tB = pairs[4 * p + 1], ncv = pairs[4 * p + 2];
   const double *VA = verts + 24 * (size_t)p, *VB = VA + 12;
   const double *cA = tetCen + 3 * tA, *cB = tetCen + 3 * tB;
   double *out = mom + 24 * (size_t)p;
-  if (ncv == 4) td_pair<4>(VA, VB, cA, cB, tp.lam[0], tp.npts[0], out, red);
-  else if (ncv == 3) td_pair<3>(VA, VB, cA, cB, tp.lam[1], tp.npts[1], out, red);
-  else td_pair<2>(VA, VB, cA, cB, tp.lam[2], tp.npts[2], out, red);
+  if (ncv == 4) td_pair<4>(VA, VB, cA, cB, td, 0, out, sh);
+  else if (ncv == 3) td_pair<3>(VA, VB, cA, cB, td, 1, out, sh);
+  else td_pair<2>(VA, VB, cA, cB, td, 2, out, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -477,34 +558,6 @@ __global__ __launch_bounds__(256) void k_fibbi(DevGeom g, const int *tdPairs, co
   for (int i = 0; i < 6; i++) table[6 * j + i] = G[i];
 }
 
-static void td_points_host(int D, int n, std::vector<double> &out)
-{
-  const int k = D - 1;
-  double gx[64], gw[64];
-  gauss01(n, gx, gw);
-  long npts = 1;
-  for (int i = 0; i < k; i++) npts *= n;
-  out.assign((size_t)(D + 1) * npts, 0.0);
-  for (long ip = 0; ip < npts; ip++) {
-    long ri = ip;
-    double t[4] = {0, 0, 0, 0}, wt = 1.0, prod = 1.0;
-    for (int d = 0; d < k; d++) {
-      int id = (int)(ri % n); ri /= n;
-      double v = gx[id];
-      prod *= v;
-      t[d] = prod;
-      for (int e = 0; e < k - 1 - d; e++) wt *= v;
-      wt *= gw[id];
-    }
-    double lam[5];
-    lam[0] = 1.0 - t[0];
-    for (int q = 1; q < k; q++) lam[q] = t[q - 1] - t[q];
-    lam[k] = t[k - 1];
-    for (int q = 0; q < D; q++) out[(size_t)q * npts + ip] = lam[q];
-    out[(size_t)D * npts + ip] = wt;
-  }
-}
-
 extern "C" int bfa_static_build(bfa_geometry *g, int td_order, void *stream)
 {
   if (!g || !g->uploaded) return fail(BFA_ERR_STATE, "bfa_static_build: geometry not uploaded");
@@ -526,20 +579,11 @@ extern "C" int bfa_static_build(bfa_geometry *g, int td_order, void *stream)
       (rc = dev_upload(&d.tdVerts, verts.data(), verts.size() * 8)) ||
       (rc = dev_upload(&d.pairTD, g->pairTD.data(), g->pairTD.size() * 4)))
     return rc;
-  // collapsed Gauss point tables for the three cases
-  const int orders[3] = {std::min(td_order + 4, 32), std::min(td_order + 2, 32), td_order};
-  const int Ds[3] = {3, 4, 5};
-  std::vector<double> tab[3];
-  void *dtab[3] = {nullptr, nullptr, nullptr};
-  TDPoints tp;
+  const int orders[3] = {std::min(td_order + 4, TD_MAXORDER), std::min(td_order + 2, TD_MAXORDER), td_order};
+  TDNodes td;
   for (int c = 0; c < 3; c++) {
-    td_points_host(Ds[c], orders[c], tab[c]);
-    if ((rc = dev_upload(&dtab[c], tab[c].data(), tab[c].size() * 8))) {
-      for (int e = 0; e < c; e++) hipFree(dtab[e]);
-      return rc;
-    }
-    tp.lam[c] = (const double *)dtab[c];
-    tp.npts[c] = (int)(tab[c].size() / (Ds[c] + 1));
+    td.n[c] = orders[c];
+    gauss01(orders[c], td.x[c], td.w[c]);
   }
   if (d.tdMom) hipFree(d.tdMom);
   d.tdMom = nullptr;
@@ -547,13 +591,10 @@ extern "C" int bfa_static_build(bfa_geometry *g, int td_order, void *stream)
   d.table = nullptr;
   hipError_t e1 = hipMalloc(&d.tdMom, std::max<size_t>(ntd, 1) * 24 * 8);
   hipError_t e2 = hipMalloc(&d.table, std::max<int64_t>(g->dg.nnz, 1) * 6 * 8);
-  if (e1 != hipSuccess || e2 != hipSuccess) {
-    for (int c = 0; c < 3; c++) hipFree(dtab[c]);
-    return fail(BFA_ERR_OOM, "bfa_static_build: allocation failed");
-  }
+  if (e1 != hipSuccess || e2 != hipSuccess) return fail(BFA_ERR_OOM, "bfa_static_build: allocation failed");
   if (ntd > 0)
     hipLaunchKernelGGL(k_td_moments, dim3((unsigned)ntd), dim3(256), 0, st, (const int *)d.tdPairs,
-                       (const double *)d.tdVerts, g->dg.tetVol + g->nt, tp, (double *)d.tdMom);
+                       (const double *)d.tdVerts, g->dg.tetVol + g->nt, td, (double *)d.tdMom);
   const int64_t nnz = g->dg.nnz;
   if (nnz > 0)
     hipLaunchKernelGGL(k_fibbi, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st, g->dg,
@@ -561,7 +602,6 @@ extern "C" int bfa_static_build(bfa_geometry *g, int td_order, void *stream)
                        (double *)d.table);
   hipError_t e3 = hipGetLastError();
   hipError_t e4 = hipStreamSynchronize(st);
-  for (int c = 0; c < 3; c++) hipFree(dtab[c]);
   if (e3 != hipSuccess || e4 != hipSuccess)
     return fail(BFA_ERR_HIP, "static build kernels failed: %s", hipGetErrorString(e3 != hipSuccess ? e3 : e4));
   g->static_built = true;
