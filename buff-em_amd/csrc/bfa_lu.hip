@@ -529,11 +529,33 @@ static void trsm(int kb, int n, const cplx<T> *L, int64_t ldl, cplx<T> *B, int64
 // workgroup owns a strip of TF_SC columns of B (column-major in LDS, 32 KB
 // so that it fits beside the trailing-update GEMM's tiles on a CU); per
 // 32-row block, the diagonal solve runs in registers (a wave takes two
-// columns, lane = row, the solved value passed along by shuffles, no
+// columns at a time, lane = row, the solved value passed along by readlane, no
 // workgroup barrier), then every row below subtracts the block's
-// contribution from register accumulators.
+// contribution from register accumulators.  Bound by the chain of the kb
+// rows: a wave with two pairs of columns solves both at once, and in complex64
+// the update's factor entries are loaded before the solve (a batch's panels:
+// 231 -> 177 us; in complex128 the 128 registers that they hold would leave one
+// wave a SIMD: 1,100 launches at n = 11,000 took 15.8 ms instead of 12.8).
 #define TF_MAXK 256
 template <typename T> struct TfShape { static constexpr int SC = 32768 / (TF_MAXK * (int)sizeof(cplx<T>)); };
+
+// v's value in lane k of the lane's half of the wavefront, by readlane: a
+// shuffle goes through LDS
+__device__ __forceinline__ float half_lane(float v, int k, int half)
+{
+  const int a = __builtin_amdgcn_readlane((int)__float_as_uint(v), k);
+  const int b = __builtin_amdgcn_readlane((int)__float_as_uint(v), k + 32);
+  return __uint_as_float((unsigned)(half ? b : a));
+}
+__device__ __forceinline__ double half_lane(double v, int k, int half)
+{
+  const int a0 = __builtin_amdgcn_readlane(__double2hiint(v), k), a1 = __builtin_amdgcn_readlane(__double2loint(v), k);
+  const int b0 = __builtin_amdgcn_readlane(__double2hiint(v), k + 32);
+  const int b1 = __builtin_amdgcn_readlane(__double2loint(v), k + 32);
+  return __hiloint2double(half ? b0 : a0, half ? b1 : a1);
+}
+template <typename T> __device__ __forceinline__ cplx<T> half_lane(cplx<T> v, int k, int half)
+{ return {half_lane(v.re, k, half), half_lane(v.im, k, half)}; }
 
 template <typename T, int SC = TfShape<T>::SC>
 __device__ __forceinline__ void trsm_lf_body(int kb, int n, const cplx<T> *__restrict__ L, int64_t ldl, cplx<T> *B,
@@ -547,33 +569,42 @@ __device__ __forceinline__ void trsm_lf_body(int kb, int n, const cplx<T> *__res
   }
   __syncthreads();
   const int row = lane & 31, half = lane >> 5;
+  constexpr int NP = SC >= 8 ? SC / 8 : 1;   // pairs of columns of a wave
   for (int b0 = 0; b0 < kb; b0 += 32) {
-    const int bk = min(32, kb - b0);
+    const int bk = min(32, kb - b0), r = b0 + bk + tid;
     cplx<T> lrow[32];
 #pragma unroll
     for (int k = 0; k < 32; k++)
       lrow[k] = (k < row && row < bk) ? L[(size_t)(b0 + k) * ldl + b0 + row] : cplx<T>{0, 0};
-    for (int pr = wave; pr < SC / 2; pr += 4) {
-      const int c = 2 * pr + half;
-      cplx<T> x = row < bk ? X[c][b0 + row] : cplx<T>{0, 0};
+    // the factor entries of the update, on their way during the solve
+    cplx<T> fr[32];
+    if (sizeof(T) == 4 && bk == 32 && r < kb) {
 #pragma unroll
-      for (int k = 0; k < 31; k++) {
-        const cplx<T> xk = {__shfl(x.re, k + 32 * half, 64), __shfl(x.im, k + 32 * half, 64)};
-        x = c_sub(x, c_mul(lrow[k], xk));   // lrow[k] = 0 unless k < row
+      for (int k = 0; k < 32; k++) fr[k] = L[(size_t)(b0 + k) * ldl + r];
+    }
+    if (2 * wave < SC) {
+      cplx<T> x[NP];
+#pragma unroll
+      for (int p = 0; p < NP; p++) x[p] = row < bk ? X[2 * (wave + 4 * p) + half][b0 + row] : cplx<T>{0, 0};
+#pragma unroll
+      for (int k = 0; k < 31; k++)
+#pragma unroll
+        for (int p = 0; p < NP; p++) x[p] = c_sub(x[p], c_mul(lrow[k], half_lane(x[p], k, half)));   // lrow[k] = 0 unless k < row
+      if (row < bk) {
+#pragma unroll
+        for (int p = 0; p < NP; p++) X[2 * (wave + 4 * p) + half][b0 + row] = x[p];
       }
-      if (row < bk) X[c][b0 + row] = x;
     }
     __syncthreads();
-    for (int r = b0 + bk + tid; r < kb; r += blockDim.x) {
+    if (r < kb) {
       cplx<T> acc[SC];
 #pragma unroll
       for (int c = 0; c < SC; c++) acc[c] = cplx<T>{0, 0};
       if (bk == 32) {
-        // a full block: the row's 32 factor entries are loaded together
-        // before use, so their latencies overlap instead of adding up
-        cplx<T> fr[32];
+        if constexpr (sizeof(T) == 8) {
 #pragma unroll
-        for (int k = 0; k < 32; k++) fr[k] = L[(size_t)(b0 + k) * ldl + r];
+          for (int k = 0; k < 32; k++) fr[k] = L[(size_t)(b0 + k) * ldl + r];
+        }
 #pragma unroll
         for (int k = 0; k < 32; k++)
 #pragma unroll
@@ -619,7 +650,8 @@ __global__ __launch_bounds__(256) void k_trsm_uf(int kb, int n, const cplx<T> *_
     X[c][r] = c < nc ? B[(size_t)(c0 + c) * ldb + r] : cplx<T>{0, 0};
   }
   __syncthreads();
-  const int row = lane & 31, half = lane >> 5;
+  const int row = lane & 31, half = lane >> 5, r = tid;
+  constexpr int NP = SC >= 8 ? SC / 8 : 1;
   for (int b0 = ((kb - 1) / 32) * 32; b0 >= 0; b0 -= 32) {
     const int bk = min(32, kb - b0);
     cplx<T> lrow[32];
@@ -627,37 +659,51 @@ __global__ __launch_bounds__(256) void k_trsm_uf(int kb, int n, const cplx<T> *_
     for (int k = 0; k < 32; k++)
       lrow[k] = (k > row && k < bk) ? U[(size_t)(b0 + k) * ldu + b0 + row] : cplx<T>{0, 0};
     const cplx<T> dinv = row < bk ? c_inv(U[(size_t)(b0 + row) * ldu + b0 + row]) : cplx<T>{0, 0};
-    for (int pr = wave; pr < SC / 2; pr += 4) {
-      const int c = 2 * pr + half;
-      cplx<T> x = row < bk ? X[c][b0 + row] : cplx<T>{0, 0};
+    cplx<T> fr[32];
+    if (sizeof(T) == 4 && bk == 32 && r < b0) {
+#pragma unroll
+      for (int k = 0; k < 32; k++) fr[k] = U[(size_t)(b0 + k) * ldu + r];
+    }
+    if (2 * wave < SC) {
+      cplx<T> x[NP];
+#pragma unroll
+      for (int p = 0; p < NP; p++) x[p] = row < bk ? X[2 * (wave + 4 * p) + half][b0 + row] : cplx<T>{0, 0};
 #pragma unroll
       for (int k = 31; k >= 0; k--) {
-        if (row == k) x = c_mul(x, dinv);
-        const cplx<T> xk = {__shfl(x.re, k + 32 * half, 64), __shfl(x.im, k + 32 * half, 64)};
-        if (row < k) x = c_sub(x, c_mul(lrow[k], xk));
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          const cplx<T> y = c_mul(x[p], dinv);
+          x[p].re = row == k ? y.re : x[p].re;
+          x[p].im = row == k ? y.im : x[p].im;
+          const cplx<T> xk = half_lane(x[p], k, half), z = c_sub(x[p], c_mul(lrow[k], xk));
+          x[p].re = row < k ? z.re : x[p].re;
+          x[p].im = row < k ? z.im : x[p].im;
+        }
       }
-      if (row < bk) X[c][b0 + row] = x;
+      if (row < bk) {
+#pragma unroll
+        for (int p = 0; p < NP; p++) X[2 * (wave + 4 * p) + half][b0 + row] = x[p];
+      }
     }
     __syncthreads();
-    for (int r = tid; r < b0; r += blockDim.x) {
+    if (r < b0) {
       cplx<T> acc[SC];
 #pragma unroll
       for (int c = 0; c < SC; c++) acc[c] = cplx<T>{0, 0};
       if (bk == 32) {
-        // a full block: the row's 32 factor entries are loaded together
-        // before use, so their latencies overlap instead of adding up
-        cplx<T> fr[32];
+        if constexpr (sizeof(T) == 8) {
 #pragma unroll
-        for (int k = 0; k < 32; k++) fr[k] = U[(size_t)(b0 + k) * ldu + r];
+          for (int k = 0; k < 32; k++) fr[k] = U[(size_t)(b0 + k) * ldu + r];
+        }
 #pragma unroll
         for (int k = 0; k < 32; k++)
 #pragma unroll
           for (int c = 0; c < SC; c++) acc[c] = c_add(acc[c], c_mul(fr[k], X[c][b0 + k]));
       } else {
         for (int k = 0; k < bk; k++) {
-          const cplx<T> u = U[(size_t)(b0 + k) * ldu + r];
+          const cplx<T> l = U[(size_t)(b0 + k) * ldu + r];
 #pragma unroll
-          for (int c = 0; c < SC; c++) acc[c] = c_add(acc[c], c_mul(u, X[c][b0 + k]));
+          for (int c = 0; c < SC; c++) acc[c] = c_add(acc[c], c_mul(l, X[c][b0 + k]));
         }
       }
 #pragma unroll
