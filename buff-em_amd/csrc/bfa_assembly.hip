@@ -75,6 +75,7 @@ static void dev_free_all(bfa::DevBuffers &d)
                    &d.tdVerts, &d.tdMom, &d.pairTD, &d.table, &d.tpTab, &d.gram};
   for (void **p : ptrs)
     if (*p) { hipFree(*p); *p = nullptr; }
+  if (d.gramEv) { (void)hipEventDestroy((hipEvent_t)d.gramEv); d.gramEv = nullptr; }
   d.tpTabBytes = 0;
 }
 
@@ -175,7 +176,9 @@ extern "C" int bfa_geometry_upload(bfa_geometry *g, void *stream)
     return rc;
   }
   if (d.gram) { hipFree(d.gram); d.gram = nullptr; }
-  if (hipMalloc(&d.gram, (size_t)std::max(nt, 1) * 16 * sizeof(cd)) != hipSuccess) {
+  if (d.gramEv) { (void)hipEventDestroy((hipEvent_t)d.gramEv); d.gramEv = nullptr; }
+  if (hipMalloc(&d.gram, (size_t)std::max(nt, 1) * 16 * sizeof(cd)) != hipSuccess ||
+      hipEventCreateWithFlags((hipEvent_t *)&d.gramEv, hipEventDisableTiming) != hipSuccess) {
     dev_free_all(d);
     return fail(BFA_ERR_OOM, "bfa_geometry_upload: allocation");
   }
@@ -1842,18 +1845,30 @@ __global__ __launch_bounds__(256) void k_near(DevGeom g, double kre, double kim,
 
 // The closed-form materials' Gram kernel is compiled without the expression
 // interpreter, whose stack is scratch memory.  kind < 0: no Gram block.
-static void launch_near(const bfa_geometry *g, double omega_re, double omega_im, const bfa_material *mat, cd *M,
+// The geometry has one set of Gram blocks, so calls on several streams or
+// threads take turns: each stream waits for the last near pass that reads
+// them.  (A captured call records no wait: its replays are ordered by whoever
+// launches them.)
+static void launch_near(bfa_geometry *g, double omega_re, double omega_im, const bfa_material *mat, cd *M,
                         int64_t ld, hipStream_t st)
 {
   const int64_t nnz = g->dg.nnz;
   cd *gram = mat->kind < 0 ? nullptr : (cd *)g->d.gram;
   if (nnz <= 0) return;
+  std::unique_lock<std::mutex> lock(g->gramMutex, std::defer_lock);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (gram) {
+    lock.lock();
+    (void)hipStreamIsCapturing(st, &cap);
+    if (cap == hipStreamCaptureStatusNone) (void)hipStreamWaitEvent(st, (hipEvent_t)g->d.gramEv, 0);
+  }
   if (gram && mat->kind == 4)
     hipLaunchKernelGGL(k_gram<true>, dim3(g->nt), dim3(64), 0, st, g->dg, omega_re, *mat, gram);
   else if (gram)
     hipLaunchKernelGGL(k_gram<false>, dim3(g->nt), dim3(64), 0, st, g->dg, omega_re, *mat, gram);
   hipLaunchKernelGGL(k_near, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st, g->dg, omega_re, omega_im,
                      (const double *)g->d.table, (const cd *)gram, M, ld);
+  if (gram && cap == hipStreamCaptureStatusNone) (void)hipEventRecord((hipEvent_t)g->d.gramEv, st);
 }
 
 // The two-pass far field's moment table (nt (nt + 1) / 2 records of 128 B,

@@ -2,6 +2,7 @@
 // kernels of the dense VIE hot path.
 #pragma once
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -57,6 +58,7 @@ struct DevBuffers {
   void *tpTab = nullptr;       // far field: 16 moments per tetrahedron pair S <= T (per frequency)
   size_t tpTabBytes = 0;
   void *gram = nullptr;        // [nt][4][4] complex Gram blocks (per frequency and material)
+  void *gramEv = nullptr;      // hipEvent_t behind the last near pass that reads them
 };
 
 }  // namespace bfa
@@ -69,6 +71,7 @@ int assemble_near_only(bfa_geometry *g, double omega_re, double omega_im, const 
 }  // namespace bfa
 
 struct bfa_geometry {
+  std::mutex gramMutex;                       // orders the calls that use d.gram
   int nv = 0, nt = 0, nbf = 0, nftot = 0;
   std::vector<double> V;                      // 3*nv
   std::vector<int> tetVI, tetFI;              // 4*nt
