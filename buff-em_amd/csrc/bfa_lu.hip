@@ -1267,8 +1267,14 @@ static int panel_regs(cplx<T> *A, int m, int w, int64_t lda, int *ipiv, int piv_
 template <typename T>
 static int lu_factor_tail(cplx<T> *A, int n, int64_t lda, int *ipiv, hipStream_t st, int j0, LUWork *lw)
 {
-  for (int j = j0; j < n; j += XP_MAXW) {
-    const int jb = std::min(XP_MAXW, n - j), next = j + jb;
+  // As few panels as XP_MAXW allows, of even width (whole 32-row blocks of the
+  // TRSM): the last panel has no TRSM and no update behind it, so a full panel
+  // and a sliver pays for a whole 256-row chain that two halves share
+  // (one right-hand side, n = 270: 256 + 14 columns 1.18 ms, 160 + 110 1.12).
+  const int np = (n - j0 + XP_MAXW - 1) / XP_MAXW;
+  const int nb = std::min(XP_MAXW, ((n - j0 + np - 1) / np + 31) / 32 * 32);
+  for (int j = j0; j < n; j += nb) {
+    const int jb = std::min(nb, n - j), next = j + jb;
     cplx<T> *Ajj = A + (size_t)j * lda + j;
     int rc = panel_regs<T>(Ajj, n - j, jb, lda, ipiv + j, j, lw, st);
     if (rc) return rc;
