@@ -722,9 +722,9 @@ __device__ __forceinline__ void tp_point_pair(const double *x, const double *y, 
 }
 
 // LDSY: the column tetrahedron's points are read from LDS (pts[1][.][ut])
-// two points at a time instead of from ys, which takes the table kernel
-// from 168 VGPRs to 122 (four waves per SIMD instead of three); the
-// single-pass kernel keeps ys (with LDSY it would spill).  The arithmetic
+// two points at a time instead of from ys, which keeps the table kernel at
+// four waves per SIMD instead of three; the single-pass kernel keeps ys (with
+// LDSY it would spill).  The arithmetic
 // and its order are the same either way; the time did not change
 // measurably (the kernel is bound by its FP64 arithmetic).
 template <bool REALK, bool LDSY = false, typename SH>
@@ -1667,7 +1667,7 @@ __device__ void overlap_entry(const DevGeom &g, int t, const double *QA, double 
 }
 
 // Eight lanes a basis function, one for each face of its two tetrahedra: with
-// one thread for all of them, 2,430 unknowns had 38 wavefronts and took
+// one thread for all of them, 2,376 unknowns had 38 wavefronts and took
 // 1.44 ms, now 0.11.  The row's first entry is the diagonal, the sum of both
 // sides; the others follow in the order of the faces.
 __global__ __launch_bounds__(128) void k_overlap_rows(DevGeom g, double omega, bfa_material mat, bfa_material temp,

@@ -535,7 +535,7 @@ static void trsm(int kb, int n, const cplx<T> *L, int64_t ldl, cplx<T> *B, int64
 // rows: a wave with two pairs of columns solves both at once, and in complex64
 // the update's factor entries are loaded before the solve (a batch's panels:
 // 231 -> 177 us; in complex128 the 128 registers that they hold would leave one
-// wave a SIMD: 1,100 launches at n = 11,000 took 15.8 ms instead of 12.8).
+// wave a SIMD: 1,100 launches at n = 11,400 took 15.8 ms instead of 12.8).
 #define TF_MAXK 256
 template <typename T> struct TfShape { static constexpr int SC = 32768 / (TF_MAXK * (int)sizeof(cplx<T>)); };
 
@@ -1796,7 +1796,7 @@ __device__ __forceinline__ cplx<T> sv_poll(const cplx<T> *p, bool act, unsigned 
 // With 4 waves that shared x through LDS (two barriers and a poll by one wave
 // a block, the product D_i^-1 L_ip formed in the sweep) a link took 6-7 us
 // with one right-hand side and 17 with eight; now 2.3 and 4.6 (complex64,
-// n = 19,440: 1.9 -> 0.69 ms a sweep, 1.5 GB of the triangle at 2.2 TB/s).
+// n = 19,872: 1.9 -> 0.69 ms a sweep, 1.6 GB of the triangle at 2.3 TB/s).
 template <typename T, bool LOWER>
 __device__ __forceinline__ void trsv_stream_body(int n, int nrhs, const cplx<T> *__restrict__ A, int64_t lda,
                                                  const cplx<T> *__restrict__ inv, const cplx<T> *Bin, cplx<T> *Xo,

@@ -282,7 +282,8 @@ int  bfa_get_fields(bfa_geometry *g, double omega, const bfa_planewave *pw, int 
  * against its complex128 matrix, then its EMT power is computed -- all in
  * grouped launches covering every instance, replayed per frequency from
  * one captured hipGraph when use_graph != 0.  Device memory per instance:
- * N*Np*16 + Np*Np*8 bytes (Np = N rounded up to 256) plus O(N) vectors.   */
+ * N*Np*16 + Np*Np*8 bytes (Np = N rounded up to 256), 2.2 MB for the LU
+ * panels' exchange, plus O(N) vectors, blocks and tetrahedron records.     */
 typedef struct bfa_batch bfa_batch;
 int  bfa_batch_create(int count, bfa_geometry *const *geoms, const bfa_material *mats,
                       const bfa_planewave *pw, int npw, bfa_batch **out);
