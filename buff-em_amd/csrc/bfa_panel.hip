@@ -21,6 +21,10 @@ template <typename T> __device__ __forceinline__ T t_fma(T a, T b, T c) { return
 // a - l u
 template <typename T> __device__ __forceinline__ zc<T> z_fms(zc<T> a, zc<T> l, zc<T> u)
 { return {t_fma(l.im, u.im, t_fma(-l.re, u.re, a.re)), t_fma(-l.im, u.re, t_fma(-l.re, u.im, a.im))}; }
+// a + l u
+template <typename T> __device__ __forceinline__ zc<T> z_fma(zc<T> a, zc<T> l, zc<T> u)
+{ return {t_fma(-l.im, u.im, t_fma(l.re, u.re, a.re)), t_fma(l.im, u.re, t_fma(l.re, u.im, a.im))}; }
+template <typename T> __device__ __forceinline__ zc<T> z_sub(zc<T> a, zc<T> b) { return {a.re - b.re, a.im - b.im}; }
 template <typename T> __device__ __forceinline__ zc<T> z_pick(bool c, zc<T> a, zc<T> b)
 { return {c ? a.re : b.re, c ? a.im : b.im}; }
 template <typename T> __device__ __forceinline__ T z_abs1(zc<T> a) { return fabs(a.re) + fabs(a.im); }
@@ -151,13 +155,30 @@ template <int LO, int HI, typename T, int R> __device__ __forceinline__ void reg
 }
 
 #define XP_NT 256
+#define XP_FOLD 32       // columns whose products are summed before they go into the values
 #define XP_SPIN_LIMIT (1u << 24)
 
-template <typename T, int NR> struct XpShared { zc<T> col[4][NR]; };
+// org: each entry's value when its sum was last zero, rows 0 .. AL - 1 (the
+// odd row length spreads a column over the banks)
+template <typename T, int R, int AL> struct XpShared {
+  zc<T> org[AL][XP_NT + 1];
+  zc<T> col[4][R];
+};
 
-// One workgroup (rank of nwg) of the panel.  Thread (h, t) holds rows
-// r0 + h R .. r0 + h R + R - 1 of column t in registers for the whole panel;
-// lanes also hold, redundantly in every wave, the next two columns row by row
+// One workgroup (rank of nwg) of the panel.  Thread t holds column t of rows
+// r0 .. r0 + R - 1 for the whole panel: in registers the sum of the products
+// l u to be subtracted from each entry, in LDS the value to subtract it from
+// (rows AL .. R - 1: in registers too).  The difference is formed where an
+// entry leaves the workgroup and every XP_FOLD columns, so an entry is rounded
+// at its own magnitude about 10 times a panel and not once a column, as with
+// the panels of 32 columns and the GEMM that accumulates from zero.
+// |PA - LU| / |A| over u, complex64, VIE matrices of 270, 1,350 and 3,822
+// unknowns: 0.82, 1.22, 1.58; subtracted from the entries product by product
+// 4.8, 7.5, 9.3, by 32-column panels 1.55, 1.87, 2.20.  On random matrices all
+// agree to 5 %; sums over the whole panel are 3 % worse there and better on
+// the VIE matrices (0.66, 1.00, 1.44).  No slower: the values, read by row
+// index, need no branch tree, and a column's time is the exchange's.
+// Lanes also hold, redundantly in every wave, the next two columns row by row
 // (lane = row), so that the multipliers of column j, the values of column
 // j + 1 and its pivot candidate need no workgroup reduction.
 //
@@ -181,37 +202,33 @@ template <typename T, int NR> struct XpShared { zc<T> col[4][NR]; };
 // step j: the interchanges of later columns are applied to them afterwards,
 // with those of the columns left of the panel (k_laswp_left); U is written at
 // the end.
-template <typename T, int WB, int R>
-__device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<T, (XP_NT / WB) * R> &sh)
+template <typename T, int R, int AL>
+__device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<T, R, AL> &sh)
 {
-  constexpr int NH = XP_NT / WB, NR = NH * R, EW = sizeof(T) / 2;   // EW: words of an entry
+  constexpr int EW = sizeof(T) / 2;   // words of an entry
+  constexpr int NX = R > AL ? R - AL : 1;
+  static_assert(R <= 64 && AL <= R, "a lane a row");
   typedef zc<T> Z;
   typedef unsigned long long u64;
   __builtin_amdgcn_s_setprio(3);
-  const int tid = threadIdx.x, lane = tid & 63, t = tid % WB;
-  const int h = __builtin_amdgcn_readfirstlane(tid / WB), t0 = __builtin_amdgcn_readfirstlane(t & ~63);
-  const int m = p.m, w = p.w, nwg = p.nwg, r0 = rank * NR;
+  const int t = threadIdx.x, lane = t & 63, t0 = __builtin_amdgcn_readfirstlane(t & ~63);
+  const int m = p.m, w = p.w, nwg = p.nwg, r0 = rank * R;
   Z *A = (Z *)p.A;
-  Z a[R];
+  Z s[R], ox[NX];
 #pragma unroll
   for (int i = 0; i < R; i++) {
-    const int r = r0 + h * R + i;
-    a[i] = (t < w && r < m) ? A[(size_t)t * p.lda + r] : Z{0, 0};
-  }
-  // columns 0, 1 to the lanes; column 2 waits in buffer 0
-  if (t < 3) {
-#pragma unroll
-    for (int i = 0; i < R; i++) sh.col[t][h * R + i] = a[i];
+    const int r = r0 + i;
+    const Z v = (t < w && r < m) ? A[(size_t)t * p.lda + r] : Z{0, 0};
+    if (i < AL) sh.org[i][t] = v;
+    else ox[i < AL ? 0 : i - AL] = v;
+    if (t < 2) sh.col[t][i] = v;   // columns 0, 1 to the lanes
+    if (t == 2) sh.col[2][i] = i < AL ? Z{0, 0} : z_sub(Z{0, 0}, v);
+    s[i] = {0, 0};
   }
   __syncthreads();
-  Z c0[NH], c1[NH], l[NH];
-#pragma unroll
-  for (int q = 0; q < NH; q++) {
-    const int i = q * R + (lane < R ? lane : 0);
-    c0[q] = sh.col[0][i];
-    c1[q] = sh.col[1][i];
-    l[q] = {0, 0};
-  }
+  const int il = lane < R ? lane : 0;
+  const bool row_lane = lane < R;
+  Z c0 = sh.col[0][il], c1 = sh.col[1][il], l = {0, 0};
   Z pt = {0, 0};
   bool dead = false;               // a wait gave up somewhere: finish without waiting
   auto wait_ok = [&](unsigned &spins) __attribute__((always_inline)) {
@@ -226,50 +243,44 @@ __device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<
   auto row_slot = [&](int buf, int who) __attribute__((always_inline)) {
     return (u64 *)p.data + ((size_t)buf * (XP_MAXWG + 1) + who) * XP_PLANE * EW;
   };
-  // row jn's register values before step jn - 1, fetched while waiting (the
-  // owner's wave half only)
-  Z xn = {0, 0};
-  auto fetch = [&](int jn) __attribute__((always_inline)) {
-    if (jn >= r0 && jn < r0 + NR && h == (jn - r0) / R) reg_get<0, R>(a, (jn - r0) % R, xn);
+  // this thread's entry of row i (wave-uniform): value, and the sum to subtract
+  auto row_get = [&](int i, Z &o, Z &q) __attribute__((always_inline)) {
+    if (AL == R || i < AL) o = sh.org[i][t];
+    else reg_get<0, NX>(ox, i - AL, o);
+    reg_get<0, R>(s, i, q);
   };
-  // row `row` of this workgroup, whose register values (x) miss step jn - 1 if elim
-  auto send = [&](int row, Z x, u64 *dst, unsigned seq, bool elim) __attribute__((always_inline)) {
-    Z lx = {0, 0};
-#pragma unroll
-    for (int q = 0; q < NH; q++)
-      if (q == h) lx = lane_get(l[q], row % R);
-    if (elim) x = z_fms(x, lx, pt);
-    put_entry(dst + t, x, seq);
+  auto row_set = [&](int i, Z v) __attribute__((always_inline)) {
+    if (AL == R || i < AL) sh.org[i][t] = v;
+    else reg_put<0, NX>(ox, i - AL, v);
+    reg_put<0, R>(s, i, Z{0, 0});
+  };
+  // row jn's entry and its sum before step jn - 1, fetched while waiting
+  Z xo = {0, 0}, xs = {0, 0};
+  auto fetch = [&](int jn) __attribute__((always_inline)) {
+    if (jn >= r0 && jn < r0 + R) row_get(jn - r0, xo, xs);
+  };
+  // row `row` of this workgroup, whose sum (q) misses step jn - 1 if elim
+  auto send = [&](int row, Z o, Z q, u64 *dst, unsigned seq, bool elim) __attribute__((always_inline)) {
+    if (elim) q = z_fma(q, lane_get(l, row), pt);
+    put_entry(dst + t, z_sub(o, q), seq);
   };
   // row jn, then the candidate of column jn (lanes hold the column in c0)
   auto publish = [&](int jn, bool elim) __attribute__((always_inline)) {
     const unsigned seq = p.seq0 + jn;
     const int buf = jn & (XP_NBUF - 1), lj = jn - r0;
-    if (lj >= 0 && lj < NR && h == lj / R) send(lj, xn, row_slot(buf, XP_MAXWG), seq, elim);
-    unsigned mg[NH], mx = 0;
-#pragma unroll
-    for (int q = 0; q < NH; q++) {
-      const int r = r0 + q * R + lane;
-      const float v = (float)z_abs1(c0[q]);
-      mg[q] = (lane < R && r < m && r >= jn) ? (v == v ? __float_as_uint(v) : 0u) + 1u : 0u;
-      mx = mg[q] > mx ? mg[q] : mx;
-    }
-    const unsigned M = wave_max(mx);
-    int rp = -1;
-    if (M) {
-#pragma unroll
-      for (int q = NH - 1; q >= 0; q--) {
-        const u64 b = __ballot(mg[q] == M);
-        if (b) rp = q * R + (int)__builtin_ctzll(b);
-      }
-    }
-    if (tid == 0)
+    if (lj >= 0 && lj < R) send(lj, xo, xs, row_slot(buf, XP_MAXWG), seq, elim);
+    const int r = r0 + lane;
+    const float v = (float)z_abs1(c0);
+    const unsigned mg = (row_lane && r < m && r >= jn) ? (v == v ? __float_as_uint(v) : 0u) + 1u : 0u;
+    const unsigned M = wave_max(mg);
+    const int rp = M ? (int)__builtin_ctzll(__ballot(mg == M)) : -1;
+    if (t == 0)
       ag_store(p.flags + ((size_t)buf * XP_MAXWG + rank) * XP_FSTRIDE,
                ((u64)seq << 40) | ((u64)M << 9) | (unsigned)(rp < 0 ? 0 : rp));
-    if (rp >= 0 && rp != lj && h == rp / R) {
-      Z x;
-      reg_get<0, R>(a, rp % R, x);
-      send(rp, x, row_slot(buf, rank), seq, elim);
+    if (rp >= 0 && rp != lj) {
+      Z o, q;
+      row_get(rp, o, q);
+      send(rp, o, q, row_slot(buf, rank), seq, elim);
     }
   };
   fetch(0);
@@ -282,7 +293,8 @@ __device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<
     // every workgroup's candidate; beside it row j, which most often is the
     // pivot's (and otherwise moves to the pivot's place): this thread's column,
     // and columns j, j + 1, j + 2 once more on lanes 0 .. 2
-    const int ib = min(j + (lane & 3), WB - 1);
+    const int ib = min(j + (lane & 3), XP_NT - 1);
+    Z ov = sh.org[AL == R ? il : min(il, AL - 1)][min(j + 2, XP_NT - 1)];   // see below
     const u64 *fl = p.flags + (size_t)buf * XP_MAXWG * XP_FSTRIDE, *rj = row_slot(buf, XP_MAXWG);
     const bool two = nwg > 64;
     u64 f, f2 = 0;
@@ -311,8 +323,8 @@ __device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<
       lrow = (int)(__builtin_amdgcn_readlane((unsigned)f2, win) & 511u);
       win = min(win + 64, nwg - 1);
     }
-    const int prow = max(j, min(m - 1, win * NR + lrow));
-    const bool ownp = prow != j && prow >= r0 && prow < r0 + NR;
+    const int prow = max(j, min(m - 1, win * R + lrow));
+    const bool ownp = prow != j && prow >= r0 && prow < r0 + R;
     Z pb = rb;
     pt = rt;
     if (prow != j) {
@@ -327,93 +339,93 @@ __device__ __forceinline__ void xpanel_body(const XPanel &p, int rank, XpShared<
     const int lp = prow - r0;
     if (prow != j) {
       const int lj = j - r0;
-      if (lj >= 0 && lj < NR && h == lj / R) reg_put<0, R>(a, lj % R, pt);
+      if (lj >= 0 && lj < R) row_set(lj, pt);
       if (ownp) {
-        if (h == lp / R) reg_put<0, R>(a, lp % R, rt);
-        if (lp == j + 1 - r0) xn = rt;
+        row_set(lp, rt);
+        if (lp == j + 1 - r0) { xo = rt; xs = {0, 0}; }
         const Z r0v = lane_get(rb, 0), r1v = lane_get(rb, 1);
-#pragma unroll
-        for (int q = 0; q < NH; q++)
-          if (q * R + lane == lp && lane < R) { c0[q] = r0v; c1[q] = r1v; }
+        if (lane == lp) { c0 = r0v; c1 = r1v; }
       }
     }
     if (t <= j) pt = {0, 0};       // finished columns: the update below leaves them alone
-    const bool scale = z_abs1(pj) != (T)0;
-    Z lo[NH];                       // column j of L as stored
-#pragma unroll
-    for (int q = 0; q < NH; q++) {
-      const bool act = lane < R && r0 + q * R + lane > j;
-      l[q] = scale && act ? z_mul(c0[q], inv) : Z{0, 0};
-      lo[q] = z_pick(scale, l[q], c0[q]);
-      c0[q] = scale && act ? z_fms(c1[q], l[q], pj1) : c1[q];
-    }
+    const bool scale = z_abs1(pj) != (T)0, act = row_lane && r0 + lane > j;
+    l = scale && act ? z_mul(c0, inv) : Z{0, 0};
+    const Z lo = z_pick(scale, l, c0);   // column j of L as stored
+    c0 = scale && act ? z_fms(c1, l, pj1) : c1;
     if (j + 1 < w) publish(j + 1, scale);
-    if ((tid >> 6) == (j & (XP_NT / 64 - 1))) {
-#pragma unroll
-      for (int q = 0; q < NH; q++) {
-        const int r = r0 + q * R + lane;
-        if (lane < R && r > j && r < m) A[(size_t)j * p.lda + r] = lo[q];
-      }
+    if ((t >> 6) == (j & (XP_NT / 64 - 1))) {
+      const int r = r0 + lane;
+      if (row_lane && r > j && r < m) A[(size_t)j * p.lda + r] = lo;
     }
-    if (rank == 0 && tid == 0) {
+    if (rank == 0 && t == 0) {
       p.ipiv[j] = prow + p.piv_off;
       if (!scale && p.err[1] == 0) p.err[1] = p.piv_off + j + 1;
     }
     __syncthreads();
-    // column j + 2 (through step j - 1) from its buffer, then step j
-#pragma unroll
-    for (int q = 0; q < NH; q++) {
-      const int i = q * R + (lane < R ? lane : 0);
-      Z v = sh.col[2 + (j & 1)][i];
-      if (ownp && i == lp) v = lane_get(rb, 2);
-      const bool act = lane < R && r0 + i > j;
-      c1[q] = scale && act ? z_fms(v, l[q], pj2) : v;
+    // column j + 2 through step j - 1, then step j.  Its thread left the sums
+    // in a buffer; the values were read from org before this step's barrier,
+    // beside which only this step's interchange may have written
+    {
+      if (AL < R && il >= AL) ov = {0, 0};
+      Z v = z_sub(ov, sh.col[2 + (j & 1)][il]);
+      if (ownp && il == lp) v = lane_get(rb, 2);
+      c1 = scale && act ? z_fms(v, l, pj2) : v;
     }
     // the other rows
-    const int ist = max(0, j + 1 - r0 - h * R);
+    const int ist = max(0, j + 1 - r0);
     if (scale && ist < R && t0 + 63 > j) {
-      Z ls = l[0];
-#pragma unroll
-      for (int q = 1; q < NH; q++)
-        if (q == h) ls = l[q];
       if (ist == 0) {
 #pragma unroll
-        for (int i = 0; i < R; i++) a[i] = z_fms(a[i], lane_get(ls, i), pt);
+        for (int i = 0; i < R; i++) s[i] = z_fma(s[i], lane_get(l, i), pt);
       } else {
 #pragma unroll
-        for (int i = 1; i < R; i++) a[i] = z_pick(i >= ist, z_fms(a[i], lane_get(ls, i), pt), a[i]);
+        for (int i = 1; i < R; i++) s[i] = z_pick(i >= ist, z_fma(s[i], lane_get(l, i), pt), s[i]);
       }
+    }
+    // every XP_FOLD columns the sums go into the values, so that neither grows long
+    if ((j & (XP_FOLD - 1)) == XP_FOLD - 1) {
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        if (i < AL) sh.org[i < AL ? i : 0][t] = z_sub(sh.org[i < AL ? i : 0][t], s[i]);
+        else ox[i < AL ? 0 : i - AL] = z_sub(ox[i < AL ? 0 : i - AL], s[i]);
+        s[i] = {0, 0};
+      }
+      __syncthreads();             // the next step's lanes read org
     }
     if (t == j + 3) {
 #pragma unroll
-      for (int i = 0; i < R; i++) sh.col[2 + ((j + 1) & 1)][h * R + i] = a[i];
+      for (int i = 0; i < R; i++)
+        sh.col[2 + ((j + 1) & 1)][i] = i < AL ? s[i] : z_sub(s[i], ox[i < AL ? 0 : i - AL]);
     }
     fetch(j + 2);
   }
 #pragma unroll
   for (int i = 0; i < R; i++) {
-    const int r = r0 + h * R + i;
-    if (t < w && r <= t && r < m) A[(size_t)t * p.lda + r] = a[i];
+    const int r = r0 + i;
+    if (t < w && r <= t && r < m)
+      A[(size_t)t * p.lda + r] = z_sub(i < AL ? sh.org[i < AL ? i : 0][t] : ox[i < AL ? 0 : i - AL], s[i]);
   }
 }
 
-template <typename T, int WB, int R> __global__ __launch_bounds__(XP_NT) void k_xpanel(XPanel p)
+template <typename T, int R> __global__ __launch_bounds__(XP_NT) void k_xpanel(XPanel p)
 {
-  __shared__ XpShared<T, (XP_NT / WB) * R> sh;
-  xpanel_body<T, WB, R>(p, blockIdx.x, sh);
+  __shared__ XpShared<T, R, R> sh;
+  xpanel_body<T, R, R>(p, blockIdx.x, sh);
 }
 
-// grouped: workgroups blk0 .. blk0 + nwg - 1 of the launch factor panel d[i]
+// grouped: workgroups blk0 .. blk0 + nwg - 1 of the launch factor panel d[i].
+// Two workgroups share a CU's LDS, so of 48 rows 38 fit in it.
 template <int R> __global__ __launch_bounds__(XP_NT) void kg_xpanel(const XPanelProb *__restrict__ d, int np)
 {
-  __shared__ XpShared<float, R> sh;
+  constexpr int AL = R < 38 ? R : 38;
+  __shared__ XpShared<float, R, AL> sh;
   int lo = 0, hi = np - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (d[mid].blk0 <= (int)blockIdx.x) lo = mid;
     else hi = mid - 1;
   }
-  xpanel_body<float, 256, R>(d[lo].p, blockIdx.x - d[lo].blk0, sh);
+  xpanel_body<float, R, AL>(d[lo].p, blockIdx.x - d[lo].blk0, sh);
 }
 
 template <int R> int resident_g()
@@ -430,10 +442,10 @@ template <int R> int resident_g()
   return n;
 }
 
-template <typename T, int WB, int R> void launch(XPanel p, hipStream_t st)
+template <typename T, int R> void launch(XPanel p, hipStream_t st)
 {
-  p.nwg = (p.m + XP_NT / WB * R - 1) / (XP_NT / WB * R);
-  hipLaunchKernelGGL((k_xpanel<T, WB, R>), dim3(p.nwg), dim3(XP_NT), 0, st, p);
+  p.nwg = (p.m + R - 1) / R;
+  hipLaunchKernelGGL((k_xpanel<T, R>), dim3(p.nwg), dim3(XP_NT), 0, st, p);
 }
 
 }  // namespace
@@ -461,15 +473,15 @@ int launch_xpanel(bool f64, XPanel p, hipStream_t st)
   if (p.m < 1 || p.m > xpanel_max_rows(f64) || p.w < 1 || p.w > XP_MAXW || p.w > p.m)
     return fail(BFA_ERR_ARG, "register panel of %d x %d", p.m, p.w);
   if (f64) {
-    if (p.m <= XP_MAXWG * 8) launch<double, 256, 8>(p, st);
-    else if (p.m <= XP_MAXWG * 16) launch<double, 256, 16>(p, st);
-    else if (p.m <= XP_MAXWG * 24) launch<double, 256, 24>(p, st);
-    else launch<double, 256, 32>(p, st);
+    if (p.m <= XP_MAXWG * 8) launch<double, 8>(p, st);
+    else if (p.m <= XP_MAXWG * 16) launch<double, 16>(p, st);
+    else if (p.m <= XP_MAXWG * 24) launch<double, 24>(p, st);
+    else launch<double, 32>(p, st);
   } else {
-    if (p.m <= XP_MAXWG * 8) launch<float, 256, 8>(p, st);
-    else if (p.m <= XP_MAXWG * 16) launch<float, 256, 16>(p, st);
-    else if (p.m <= XP_MAXWG * 32) launch<float, 256, 32>(p, st);
-    else launch<float, 256, 48>(p, st);
+    if (p.m <= XP_MAXWG * 8) launch<float, 8>(p, st);
+    else if (p.m <= XP_MAXWG * 16) launch<float, 16>(p, st);
+    else if (p.m <= XP_MAXWG * 32) launch<float, 32>(p, st);
+    else launch<float, 48>(p, st);
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? BFA_OK : fail(BFA_ERR_HIP, "register panel launch: %s", hipGetErrorString(e));

@@ -181,3 +181,35 @@ def test_batch_single_pass_far_field(bfa, torch_cuda, batch_setup, tmp_path):
         assert err < 1e-14
     rel = np.abs(two["power"] - single["power"]) / np.abs(single["power"])
     assert rel.max() < 1e-12, rel.max()
+
+
+def test_batch_tall_panels(bfa, torch_cuda):
+    """More rows than 32 for each of a panel's 128 workgroups (N = 5,760, the
+    variant of 48 whose last rows lie outside LDS), beside a small instance:
+    the complex64 factors precondition as well as the single path's."""
+    torch = torch_cuda
+    geoms, mats = [], []
+    for n, seed in ((8, 21), (3, 22)):
+        V, T = bfa.kuhn_sphere(n, 0.9, 0.05, seed)
+        g = bfa.Geometry(V, T)
+        g.upload()
+        g.build_static(6)
+        geoms.append(g)
+        mats.append(bfa.material("janus", up=4 + 0.1j, down=12 + 1j))
+    pws = bfa.planewaves(SPEC[:1])
+    r = bfa.Batch(geoms, mats, pws).run([1.5], use_graph=False)
+    assert (r["info"] == 0).all()
+    for i, (g, m) in enumerate(zip(geoms, mats)):
+        M = torch.empty((g.N, g.N), dtype=torch.complex128, device="cuda:0")
+        B = torch.empty((1, g.N), dtype=torch.complex128, device="cuda:0")
+        piv = torch.empty(g.N, dtype=torch.int32, device="cuda:0")
+        g.assemble_vie(1.5, m, M)
+        g.assemble_rhs(1.5, pws, B)
+        M32 = torch.empty((g.N, g.N), dtype=torch.complex64, device="cuda:0")
+        bfa.convert_z2c(M, g.N, g.N, M32)
+        assert bfa.lu_factor_c(M32, g.N, piv) == 0
+        it, res = bfa.solve_refine(M, M32, piv, g.N, B, 1, tol=1e-10, maxit=10)
+        P = g.emt_power(1.5, pws, B)
+        # both refined to 1e-10, and one step of slack for another rounding
+        assert np.abs(r["power"][0, i] - P).max() <= 1e-9 * np.abs(P).max()
+        assert r["iters"][0, i] <= it + 1
