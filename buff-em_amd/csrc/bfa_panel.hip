@@ -72,8 +72,9 @@ __device__ __forceinline__ bool get_entry(const unsigned long long *p, zc<float>
   return (unsigned)(a >> 32) == seq && (unsigned)(b >> 32) == seq;
 }
 // 1 / a: on the path from one exchange to the next, so the reciprocal of
-// |a|^2 comes from the hardware estimate and two Newton steps where that
-// cannot overflow, in place of two divisions
+// |a|^2 comes from the hardware estimate and Newton steps where that cannot
+// overflow, and each quotient is corrected by its own remainder: as exact as
+// the two divisions it stands for
 __device__ __forceinline__ double recip(double d)
 {
   double y = __builtin_amdgcn_rcp(d);
@@ -90,8 +91,8 @@ template <typename T> __device__ __forceinline__ zc<T> z_inv(zc<T> a)
   constexpr T big = sizeof(T) == 8 ? (T)1e290 : (T)1e30;
   const T d = a.re * a.re + a.im * a.im;
   if (d > 1 / big && d < big) {
-    const T y = recip(d);
-    return {a.re * y, -a.im * y};
+    const T y = recip(d), p = a.re * y, q = -a.im * y;
+    return {t_fma(y, t_fma(-d, p, a.re), p), t_fma(y, t_fma(-d, q, -a.im), q)};
   }
   return {a.re / d, -a.im / d};
 }

@@ -108,3 +108,33 @@ def test_panel_factor_error_without_interchanges(n, f64):
         err = (torch.linalg.norm(MM - L @ torch.triu(LU)) / torch.linalg.norm(MM)).item()
     u = np.finfo(np.float64 if f64 else np.float32).eps / 2
     assert err <= 3 * u
+
+
+@pytest.mark.gpu
+def test_panel_multiplier_is_as_exact_as_division():
+    """l = a / p by the pivot's inverse: against the same formula in float with
+    IEEE divisions, |p|^2 without and the product with fused multiply-adds
+    (which of them the compiler fuses is its choice)."""
+    bfa = _load()
+    rng = np.random.default_rng(1)
+    f = np.float32
+    got, ref = [], []
+    for _ in range(600):
+        M = (rng.standard_normal((2, 2)) + 1j * rng.standard_normal((2, 2))) * np.exp(rng.uniform(-3, 3))
+        M[0] *= 3
+        M = M.astype(np.complex64)
+        A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+        info, piv = _factor(bfa, A, False)
+        assert info == 0
+        a, p = (M[1, 0], M[0, 0]) if piv[0] == 0 else (M[0, 0], M[1, 0])
+        # float products are exact in double: one rounding each
+        d = f(f(p.real * p.real) + f(p.imag * p.imag))
+        v = [np.float64(f(p.real / d)), np.float64(f(-p.imag / d))]
+        ar, ai = np.float64(a.real), np.float64(a.imag)
+        want = complex(f(ar * v[0] - f(ai * v[1])), f(ar * v[1] + f(ai * v[0])))
+        exact = complex(a) / complex(p)
+        got.append(abs(complex(A.cpu().numpy()[0, 1]) - exact) / abs(exact))
+        ref.append(abs(want - exact) / abs(exact))
+    rms = lambda e: np.sqrt(np.mean(np.square(e)))
+    # 0.84 u against 0.87 u on the same samples; 0.94 u with products by an inverse rounded once more
+    assert rms(got) <= rms(ref)
