@@ -641,7 +641,7 @@ struct Planner {
     return BFA_OK;
   }
 
-  // 256-column panels of up to xpanel_max_rows rows: register panels, as many
+  // 256-column panels of up to xpanel_group_max_rows rows: register panels, as many
   // to a launch as may run at once
   int panel_regs(const std::vector<Pan> &ps)
   {
@@ -683,6 +683,7 @@ struct Planner {
   int lu()
   {
     int maxNp = 0;
+    const int xrows = xpanel_group_max_rows();
     for (int i = 0; i < B->count; i++) maxNp = std::max(maxNp, B->Np[i]);
     for (int j = 0; j < maxNp; j += NB) {
       std::vector<Pan> ps;
@@ -693,7 +694,7 @@ struct Planner {
         ps.push_back({A + (size_t)j * ld + j, ld, B->Np[i] - j, B->ipiv(i) + j, j, i});
       }
       std::vector<Pan> tall, low;
-      for (const Pan &p : ps) (p.m > xpanel_max_rows(false) ? tall : low).push_back(p);
+      for (const Pan &p : ps) (p.m > xrows ? tall : low).push_back(p);
       int rc = BFA_OK;
       if (!tall.empty()) rc = panel_rec(tall, NB);
       if (!rc && !low.empty()) rc = panel_regs(low);
@@ -710,7 +711,7 @@ struct Planner {
         SwapProb s{};
         s.A = A; s.ipiv = ip; s.lda = p.lda; s.c0 = 0; s.c1 = j; s.k0 = j; s.kb = NB;
         // a register panel leaves its multipliers in the rows of their step
-        if (p.m <= xpanel_max_rows(false)) { s.own = 1; s.c1 = j + NB; }
+        if (p.m <= xrows) { s.own = 1; s.c1 = j + NB; }
         sw.push_back(s);
         s.own = 0;
         s.c0 = j + NB; s.c1 = B->Np[i];

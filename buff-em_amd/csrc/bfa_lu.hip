@@ -1257,6 +1257,19 @@ static int panel_regs(cplx<T> *A, int m, int w, int64_t lda, int *ipiv, int piv_
   return launch_xpanel(sizeof(T) == 8, p, st);
 }
 
+// Tallest register panel on stream st.  On a stream that owns only part of the
+// CUs its workgroups may not all run at once, even where their number fits:
+// they are dealt in turn to each XCD's shader engines, whatever CUs those
+// have.  Such a stream takes the panels of few workgroups.
+static int tail_rows(bool f64, hipStream_t st, const LUWork *lw)
+{
+  uint32_t mask[32] = {};
+  int cus = 0;
+  if (hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) (void)hipGetLastError();
+  for (uint32_t m : mask) cus += __builtin_popcount(m);
+  return cus > 0 && cus < lw->num_cu ? 0 : xpanel_max_rows(f64);
+}
+
 // Columns [j0, n) of a matrix whose remaining rows fit the register panel, on
 // one stream: a 256-column panel costs ~2 us a column whatever its height,
 // against ~5 us a column plus seven TRSM / GEMM / swap launches per 256
@@ -1356,7 +1369,7 @@ static int lu_factor_masked(cplx<T> *A, int n, int64_t lda, int *ipiv, int *info
   int rc = panel_rec<T>(A, n, std::min(nb, n), lda, ipiv, 0, lw, sp, P);
   if (rc) return rc;
   bool sliced = false;                           // the panel stream updated a column slice last step
-  const int cap = xpanel_max_rows(sizeof(T) == 8);
+  const int cap = tail_rows(sizeof(T) == 8, st, lw);
   int tail = n;
   for (int j = 0; j < n; j += nb) {
     const int jb = std::min(nb, n - j);
@@ -1440,8 +1453,7 @@ int lu_factor(cplx<T> *A, int n, int64_t lda, int *ipiv, int *info, hipStream_t 
   LUWork *lw = nullptr;
   int rc = lu_work(lw);
   if (rc) return rc;
-  const int cap = xpanel_max_rows(sizeof(T) == 8);
-  if (n <= cap) {
+  if (n <= tail_rows(sizeof(T) == 8, st, lw)) {
     HIPCHECK(hipMemsetAsync(lw->pw.flags, 0, 8, st));
     if ((rc = lu_factor_tail<T>(A, n, lda, ipiv, st, 0, lw))) return rc;
     return lu_flags(lw, info, st);

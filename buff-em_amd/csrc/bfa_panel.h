@@ -24,6 +24,7 @@ struct XPanel {
 // exchange memory of one panel at a time: bytes, and its division
 size_t xpanel_bytes(bool f64);
 void xpanel_carve(bool f64, char *mem, XPanel *p);
+// tallest panel whose workgroups run at once on the current device (0: none)
 int xpanel_max_rows(bool f64);
 int launch_xpanel(bool f64, XPanel p, hipStream_t st);
 
@@ -36,5 +37,11 @@ struct XPanelProb {
 // rows a workgroup for panels of at most m rows that fill `total` rows in all,
 // and the workgroups that may run at once with it (0: none)
 int xpanel_group_rows(int m, int64_t total, int *resident);
+// tallest panel of a grouped launch (0: none)
+int xpanel_group_max_rows();
 void launch_xpanel_g(const XPanelProb *d, int np, int nblk, int rows, hipStream_t st);
 }  // namespace bfa
+
+// rows a workgroup for a panel of m rows where per_cu[v] workgroups of variant v
+// (fewest rows first, four of them) run on each of `cus` CUs; 0: none fits
+extern "C" int bfa_xpanel_rows(int f64, int m, int cus, const int *per_cu);

@@ -6,6 +6,7 @@
 // (src/applications/buff-scatter/buff-scatter.cc:285).
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <mutex>
 
 #include "bfa_internal.h"
 #include "bfa_panel.h"
@@ -429,18 +430,42 @@ template <int R> __global__ __launch_bounds__(XP_NT) void kg_xpanel(const XPanel
   xpanel_body<float, R, AL>(d[lo].p, blockIdx.x - d[lo].blk0, sh);
 }
 
-template <int R> int resident_g()
+const int g_rows[2][4] = {{8, 16, 32, 48}, {8, 16, 24, 32}};   // [f64]
+const int g_group_rows[3] = {16, 32, 48};
+
+// workgroups of each variant on one CU, and the CUs, of the current device
+struct Occupancy { int cus, per[2][4], group[3]; };
+const Occupancy &occupancy()
 {
-  static int n = -1;
-  if (n < 0) {
-    int per = 0, dev = 0;
-    hipDeviceProp_t prop;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kg_xpanel<R>, XP_NT, 0) != hipSuccess ||
-        hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
-      per = 0;
-    n = per > 0 ? std::min(per, 2) * prop.multiProcessorCount : 0;
-  }
-  return n;
+  static Occupancy none{}, tab[16];
+  static bool have[16];
+  static std::mutex mx;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return none;
+  std::lock_guard<std::mutex> lock(mx);
+  Occupancy &o = tab[dev];
+  if (have[dev]) return o;
+  const void *k[2][4] = {
+      {(const void *)k_xpanel<float, 8>, (const void *)k_xpanel<float, 16>, (const void *)k_xpanel<float, 32>,
+       (const void *)k_xpanel<float, 48>},
+      {(const void *)k_xpanel<double, 8>, (const void *)k_xpanel<double, 16>, (const void *)k_xpanel<double, 24>,
+       (const void *)k_xpanel<double, 32>}};
+  const void *kg[3] = {(const void *)kg_xpanel<16>, (const void *)kg_xpanel<32>, (const void *)kg_xpanel<48>};
+  auto count = [](const void *f) {
+    int per = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, f, XP_NT, 0) == hipSuccess ? per : 0;
+  };
+  if (hipDeviceGetAttribute(&o.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return none;
+  for (int v = 0; v < 4; v++) { o.per[0][v] = count(k[0][v]); o.per[1][v] = count(k[1][v]); }
+  for (int v = 0; v < 3; v++) o.group[v] = count(kg[v]);
+  have[dev] = true;
+  return o;
+}
+// workgroups of a grouped launch: two a CU at most
+int resident_g(int v)
+{
+  const Occupancy &o = occupancy();
+  return std::min(o.group[v], 2) * o.cus;
 }
 
 template <typename T, int R> void launch(XPanel p, hipStream_t st)
@@ -467,21 +492,31 @@ void xpanel_carve(bool f64, char *mem, XPanel *p)
 // column of 256: complex128 1.76 (8 rows, m = 256), 1.99 (16, 1,350), 2.4
 // (24, 3,000), 2.6 (32, 1,350); complex64 1.53 (8, 256), 1.73 (16, 1,350),
 // 2.2 (32, 4,000), 2.6 (48, 6,000).
-int xpanel_max_rows(bool f64) { return XP_MAXWG * (f64 ? 32 : 48); }
+// A panel's workgroups wait for each other, so all must run at once: XP_MAXWG
+// of them at most, and what the device holds (a partition of it has fewer CUs).
+int xpanel_max_rows(bool f64)
+{
+  const Occupancy &o = occupancy();
+  int rows = 0;
+  for (int v = 0; v < 4; v++) rows = std::max(rows, g_rows[f64][v] * std::min(XP_MAXWG, o.per[f64][v] * o.cus));
+  return rows;
+}
 
 int launch_xpanel(bool f64, XPanel p, hipStream_t st)
 {
-  if (p.m < 1 || p.m > xpanel_max_rows(f64) || p.w < 1 || p.w > XP_MAXW || p.w > p.m)
+  const Occupancy &o = occupancy();
+  const int rows = bfa_xpanel_rows(f64, p.m, o.cus, o.per[f64]);
+  if (p.m < 1 || !rows || p.w < 1 || p.w > XP_MAXW || p.w > p.m)
     return fail(BFA_ERR_ARG, "register panel of %d x %d", p.m, p.w);
   if (f64) {
-    if (p.m <= XP_MAXWG * 8) launch<double, 8>(p, st);
-    else if (p.m <= XP_MAXWG * 16) launch<double, 16>(p, st);
-    else if (p.m <= XP_MAXWG * 24) launch<double, 24>(p, st);
+    if (rows == 8) launch<double, 8>(p, st);
+    else if (rows == 16) launch<double, 16>(p, st);
+    else if (rows == 24) launch<double, 24>(p, st);
     else launch<double, 32>(p, st);
   } else {
-    if (p.m <= XP_MAXWG * 8) launch<float, 8>(p, st);
-    else if (p.m <= XP_MAXWG * 16) launch<float, 16>(p, st);
-    else if (p.m <= XP_MAXWG * 32) launch<float, 32>(p, st);
+    if (rows == 8) launch<float, 8>(p, st);
+    else if (rows == 16) launch<float, 16>(p, st);
+    else if (rows == 32) launch<float, 32>(p, st);
     else launch<float, 48>(p, st);
   }
   const hipError_t e = hipGetLastError();
@@ -492,15 +527,21 @@ int launch_xpanel(bool f64, XPanel p, hipStream_t st)
 // grows with the rows, see above, and with a second round of launches more)
 int xpanel_group_rows(int m, int64_t total, int *resident)
 {
-  const int rows[3] = {16, 32, 48}, res[3] = {resident_g<16>(), resident_g<32>(), resident_g<48>()};
   int pick = -1;
   for (int i = 0; i < 3; i++) {
-    if (m > rows[i] * XP_MAXWG || res[i] < XP_MAXWG) continue;
+    if (m > g_group_rows[i] * std::min(XP_MAXWG, resident_g(i))) continue;
     pick = i;
-    if (total <= (int64_t)rows[i] * res[i]) break;
+    if (total <= (int64_t)g_group_rows[i] * resident_g(i)) break;
   }
-  *resident = pick < 0 ? 0 : res[pick];
-  return pick < 0 ? 0 : rows[pick];
+  *resident = pick < 0 ? 0 : resident_g(pick);
+  return pick < 0 ? 0 : g_group_rows[pick];
+}
+
+int xpanel_group_max_rows()
+{
+  int rows = 0;
+  for (int i = 0; i < 3; i++) rows = std::max(rows, g_group_rows[i] * std::min(XP_MAXWG, resident_g(i)));
+  return rows;
 }
 
 void launch_xpanel_g(const XPanelProb *d, int np, int nblk, int rows, hipStream_t st)
@@ -511,3 +552,11 @@ void launch_xpanel_g(const XPanelProb *d, int np, int nblk, int rows, hipStream_
   else hipLaunchKernelGGL(kg_xpanel<48>, dim3(nblk), dim3(XP_NT), 0, st, d, np);
 }
 }  // namespace bfa
+
+extern "C" int bfa_xpanel_rows(int f64, int m, int cus, const int *per_cu)
+{
+  const int *rows = g_rows[f64 ? 1 : 0];
+  for (int v = 0; v < 4; v++)
+    if (m <= rows[v] * std::min(XP_MAXWG, per_cu[v] * cus)) return rows[v];
+  return 0;
+}

@@ -138,3 +138,51 @@ def test_panel_multiplier_is_as_exact_as_division():
     rms = lambda e: np.sqrt(np.mean(np.square(e)))
     # 0.84 u against 0.87 u on the same samples; 0.94 u with products by an inverse rounded once more
     assert rms(got) <= rms(ref)
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+def test_panel_workgroups_run_at_once(f64):
+    """The variant of a panel: fewest rows whose workgroups, which wait for each
+    other, all fit -- 128 of them, and what the CUs hold."""
+    import ctypes
+    lib = _load().lib()
+    variants = [8, 16, 24, 32] if f64 else [8, 16, 32, 48]
+    for cus in (1, 4, 16, 32, 64, 128, 256):
+        for per in ([4, 2, 1, 1], [7, 4, 2, 1], [1, 1, 1, 1], [1, 1, 0, 0], [0, 0, 0, 0]):
+            arr = (ctypes.c_int * 4)(*per)
+            for m in (1, 8, 9, 255, 256, 270, 1024, 1025, 2048, 2049, 3072, 3073, 4096, 4097, 6144, 6145):
+                rows = lib.bfa_xpanel_rows(f64, m, cus, arr)
+                fits = [r for r, p in zip(variants, per) if -(-m // r) <= min(128, p * cus)]
+                assert rows == (fits[0] if fits else 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f64", [True, False])
+def test_panel_on_a_stream_with_part_of_the_cus(f64):
+    """A caller's stream that owns 32 CUs: 1,350 rows would take 85 workgroups."""
+    import ctypes
+    bfa = _load()
+    torch.zeros(1, device="cuda")
+    hip = ctypes.CDLL("libamdhip64.so")
+    mask = (ctypes.c_uint32 * 8)(0xFFFFFFFF)
+    h = ctypes.c_void_p()
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(h), 8, mask) == 0
+    st = torch.cuda.ExternalStream(h.value)
+    n = 1350
+    rng = np.random.default_rng(2)
+    M = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))).astype(np.complex128 if f64 else np.complex64)
+    A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+    piv = torch.zeros(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    assert (bfa.lu_factor if f64 else bfa.lu_factor_c)(A, n, piv, stream=st) == 0
+    torch.cuda.synchronize()
+    LU = A.T.to(torch.complex128)
+    L, U = torch.tril(LU, -1) + torch.eye(n, dtype=LU.dtype, device="cuda"), torch.triu(LU)
+    perm = np.arange(n)
+    for i, p in enumerate(piv.cpu().numpy()):
+        perm[[i, p]] = perm[[p, i]]
+    PA = torch.from_numpy(M[perm].astype(np.complex128)).cuda()
+    u = np.finfo(np.float64 if f64 else np.float32).eps / 2
+    # |PA - LU| <= gamma_n |L||U|, as above
+    assert torch.linalg.norm(PA - L @ U) <= n * np.sqrt(8.0) * u * torch.linalg.norm(L.abs() @ U.abs())
+    assert hip.hipStreamDestroy(h) == 0
