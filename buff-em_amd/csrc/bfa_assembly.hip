@@ -75,7 +75,7 @@ static void dev_free_all(bfa::DevBuffers &d)
                    &d.tdVerts, &d.tdMom, &d.pairTD, &d.table, &d.tpTab, &d.gram};
   for (void **p : ptrs)
     if (*p) { hipFree(*p); *p = nullptr; }
-  if (d.gramEv) { (void)hipEventDestroy((hipEvent_t)d.gramEv); d.gramEv = nullptr; }
+  if (d.turnEv) { (void)hipEventDestroy((hipEvent_t)d.turnEv); d.turnEv = nullptr; }
   d.tpTabBytes = 0;
 }
 
@@ -176,9 +176,9 @@ extern "C" int bfa_geometry_upload(bfa_geometry *g, void *stream)
     return rc;
   }
   if (d.gram) { hipFree(d.gram); d.gram = nullptr; }
-  if (d.gramEv) { (void)hipEventDestroy((hipEvent_t)d.gramEv); d.gramEv = nullptr; }
+  if (d.turnEv) { (void)hipEventDestroy((hipEvent_t)d.turnEv); d.turnEv = nullptr; }
   if (hipMalloc(&d.gram, (size_t)std::max(nt, 1) * 16 * sizeof(cd)) != hipSuccess ||
-      hipEventCreateWithFlags((hipEvent_t *)&d.gramEv, hipEventDisableTiming) != hipSuccess) {
+      hipEventCreateWithFlags((hipEvent_t *)&d.turnEv, hipEventDisableTiming) != hipSuccess) {
     dev_free_all(d);
     return fail(BFA_ERR_OOM, "bfa_geometry_upload: allocation");
   }
@@ -1843,32 +1843,42 @@ __global__ __launch_bounds__(256) void k_near(DevGeom g, double kre, double kim,
   if (j < g.nnz) near_entry(g, kre, kim, table, gram, M, ld, j);
 }
 
+// The geometry has one moment table and one set of Gram blocks, for one
+// frequency and one material, so assemblies of it on several streams or
+// threads take turns: one call at a time is put on its stream, which waits for
+// the last call's kernels.  (A captured call records no wait: its replays are
+// ordered by whoever launches them.)
+struct AssemblyTurn {
+  bfa_geometry *g;
+  hipStream_t st;
+  std::lock_guard<std::mutex> lock;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  AssemblyTurn(bfa_geometry *g, hipStream_t st) : g(g), st(st), lock(g->turn)
+  {
+    (void)hipStreamIsCapturing(st, &cap);
+    if (cap == hipStreamCaptureStatusNone) (void)hipStreamWaitEvent(st, (hipEvent_t)g->d.turnEv, 0);
+  }
+  ~AssemblyTurn()
+  {
+    if (cap == hipStreamCaptureStatusNone) (void)hipEventRecord((hipEvent_t)g->d.turnEv, st);
+  }
+};
+
 // The closed-form materials' Gram kernel is compiled without the expression
 // interpreter, whose stack is scratch memory.  kind < 0: no Gram block.
-// The geometry has one set of Gram blocks, so calls on several streams or
-// threads take turns: each stream waits for the last near pass that reads
-// them.  (A captured call records no wait: its replays are ordered by whoever
-// launches them.)
+// Called within the geometry's AssemblyTurn.
 static void launch_near(bfa_geometry *g, double omega_re, double omega_im, const bfa_material *mat, cd *M,
                         int64_t ld, hipStream_t st)
 {
   const int64_t nnz = g->dg.nnz;
   cd *gram = mat->kind < 0 ? nullptr : (cd *)g->d.gram;
   if (nnz <= 0) return;
-  std::unique_lock<std::mutex> lock(g->gramMutex, std::defer_lock);
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (gram) {
-    lock.lock();
-    (void)hipStreamIsCapturing(st, &cap);
-    if (cap == hipStreamCaptureStatusNone) (void)hipStreamWaitEvent(st, (hipEvent_t)g->d.gramEv, 0);
-  }
   if (gram && mat->kind == 4)
     hipLaunchKernelGGL(k_gram<true>, dim3(g->nt), dim3(64), 0, st, g->dg, omega_re, *mat, gram);
   else if (gram)
     hipLaunchKernelGGL(k_gram<false>, dim3(g->nt), dim3(64), 0, st, g->dg, omega_re, *mat, gram);
   hipLaunchKernelGGL(k_near, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st, g->dg, omega_re, omega_im,
                      (const double *)g->d.table, (const cd *)gram, M, ld);
-  if (gram && cap == hipStreamCaptureStatusNone) (void)hipEventRecord((hipEvent_t)g->d.gramEv, st);
 }
 
 // The two-pass far field's moment table (nt (nt + 1) / 2 records of 128 B,
@@ -1913,6 +1923,7 @@ static int assemble_vie(bfa_geometry *g, double omega_re, double omega_im, const
   const int nt2 = (N + FT2 - 1) / FT2;
   const int64_t nblk2 = (int64_t)nt2 * (nt2 + 1) / 2;
   const bool rk = omega_im == 0.0;
+  AssemblyTurn turn(g, st);
   double *tpt = far_table(g);
   if (tpt) {
     const int ntb = (g->nt + 31) / 32;
@@ -1972,6 +1983,7 @@ int bfa::assemble_near_only(bfa_geometry *g, double omega_re, double omega_im, c
 {
   if (!g || !mat || !d_M) return fail(BFA_ERR_ARG, "assemble_near_only: null argument");
   if (!g->uploaded || !g->static_built) return fail(BFA_ERR_STATE, "assemble_near_only: static table not built");
+  AssemblyTurn turn(g, (hipStream_t)stream);
   launch_near(g, omega_re, omega_im, mat, (cd *)d_M, ld, (hipStream_t)stream);
   HIPCHECK(hipGetLastError());
   return BFA_OK;

@@ -58,7 +58,7 @@ struct DevBuffers {
   void *tpTab = nullptr;       // far field: 16 moments per tetrahedron pair S <= T (per frequency)
   size_t tpTabBytes = 0;
   void *gram = nullptr;        // [nt][4][4] complex Gram blocks (per frequency and material)
-  void *gramEv = nullptr;      // hipEvent_t behind the last near pass that reads them
+  void *turnEv = nullptr;      // hipEvent_t behind the last assembly that uses tpTab and gram
 };
 
 }  // namespace bfa
@@ -71,7 +71,7 @@ int assemble_near_only(bfa_geometry *g, double omega_re, double omega_im, const 
 }  // namespace bfa
 
 struct bfa_geometry {
-  std::mutex gramMutex;                       // orders the calls that use d.gram
+  std::mutex turn;                            // held while an assembly is put on its stream
   int nv = 0, nt = 0, nbf = 0, nftot = 0;
   std::vector<double> V;                      // 3*nv
   std::vector<int> tetVI, tetFI;              // 4*nt
