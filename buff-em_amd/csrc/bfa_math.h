@@ -17,10 +17,12 @@ __device__ __forceinline__ double rsqrt_nr(double x)
 }
 
 // sin and cos of a phase k r: reduced by multiples n of pi/2, which two doubles
-// hold to 2^-109 (n times that stays below rounding up to |x| = 2^50, far
-// beyond any phase whose own rounding leaves it a meaning), then the Taylor
-// polynomials on |f| <= pi/4, whose first dropped terms are f^17/17! <= 5e-17
-// and f^18/18! <= 2e-18.  About 30 instructions, no table and no branch,
+// hold to 2^-109, then the Taylor polynomials on |f| <= pi/4, whose first
+// dropped terms are f^17/17! <= 5e-17 and f^18/18! <= 2e-18.  That |f| takes
+// n = x 2/pi to within rounding of the nearest: true to 0.002 for |x| < 2^44.
+// Above, the product's rounding moves n, |f| reaches 0.95 and the dropped term
+// 1.2e-15 at 2^50, where x's own last place is already 0.25; larger phases
+// carry no digits and get none here.  About 30 instructions, no table and no branch,
 // against some 80 and twice the registers with the library's sincos and its
 // reduction for huge arguments.
 __device__ __forceinline__ void sincos_mod(double x, double *sn, double *cs)
