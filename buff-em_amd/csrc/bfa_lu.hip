@@ -2218,6 +2218,15 @@ void launch_panel_g(bool f64, const PanelProb *d, int np, int nblk, size_t lds, 
 }  // namespace bfa
 
 // ---------------------------------------------------------------------------
+extern "C" unsigned bfa_xpanel_seq(unsigned seq)
+{
+  bfa::LUWork *lw = nullptr;
+  if (bfa::lu_work(lw)) return 0;
+  // never back: words of a number used before would look current
+  lw->xseq = std::max(lw->xseq, std::min(seq, (1u << 24) - 1));
+  return lw->xseq;
+}
+
 extern "C" int bfa_lu_factor_z(void *d_A, int n, int64_t lda, int *d_ipiv, int *info, void *stream)
 {
   if (!d_A || !d_ipiv || n <= 0 || lda < n) return fail(BFA_ERR_ARG, "bfa_lu_factor_z: bad argument");

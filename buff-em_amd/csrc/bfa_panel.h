@@ -42,6 +42,9 @@ int xpanel_group_max_rows();
 void launch_xpanel_g(const XPanelProb *d, int np, int nblk, int rows, hipStream_t st);
 }  // namespace bfa
 
+// moves the device's panel sequence numbers forward (tests of their restart);
+// returns the next one to be used
+extern "C" unsigned bfa_xpanel_seq(unsigned seq);
 // rows a workgroup for a panel of m rows where per_cu[v] workgroups of variant v
 // (fewest rows first, four of them) run on each of `cus` CUs; 0: none fits
 extern "C" int bfa_xpanel_rows(int f64, int m, int cus, const int *per_cu);

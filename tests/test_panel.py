@@ -1,6 +1,7 @@
 """Register-resident LU panel (bfa_panel.hip) at the sizes where its workgroup
 shape changes: one row, the edges of a 256-column panel, the first size of each
-rows-a-workgroup variant, and the largest matrix that takes it whole."""
+rows-a-workgroup variant, and the largest matrix that takes it whole (4,096 rows
+in complex128, 6,144 in complex64: every workgroup full)."""
 import numpy as np
 import pytest
 
@@ -176,13 +177,73 @@ def test_panel_on_a_stream_with_part_of_the_cus(f64):
     torch.cuda.synchronize()
     assert (bfa.lu_factor if f64 else bfa.lu_factor_c)(A, n, piv, stream=st) == 0
     torch.cuda.synchronize()
+    _check_factors(M, A, piv.cpu().numpy(), f64)
+    assert hip.hipStreamDestroy(h) == 0
+
+
+def _check_factors(M, A, piv, f64):
+    n = len(M)
     LU = A.T.to(torch.complex128)
-    L, U = torch.tril(LU, -1) + torch.eye(n, dtype=LU.dtype, device="cuda"), torch.triu(LU)
+    L = torch.tril(LU, -1) + torch.eye(n, dtype=LU.dtype, device="cuda")
+    U = torch.triu(LU)
     perm = np.arange(n)
-    for i, p in enumerate(piv.cpu().numpy()):
+    for i, p in enumerate(piv):
+        assert i <= p < n
         perm[[i, p]] = perm[[p, i]]
     PA = torch.from_numpy(M[perm].astype(np.complex128)).cuda()
+    # |PA - LU| <= gamma_n |L||U| entry by entry, gamma_n = n sqrt(8) u for complex arithmetic; in norms
     u = np.finfo(np.float64 if f64 else np.float32).eps / 2
-    # |PA - LU| <= gamma_n |L||U|, as above
-    assert torch.linalg.norm(PA - L @ U) <= n * np.sqrt(8.0) * u * torch.linalg.norm(L.abs() @ U.abs())
-    assert hip.hipStreamDestroy(h) == 0
+    bound = n * np.sqrt(8.0) * u * torch.linalg.norm(L.abs() @ U.abs())
+    assert torch.linalg.norm(PA - L @ U) <= bound
+    # partial pivoting: no multiplier is larger than its pivot in |re| + |im| (izamax's norm): |l| <= sqrt(2),
+    # and the float rounding of the compared magnitudes
+    assert L.abs().max() <= np.sqrt(2.0) * (1 + 1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,f64", [(4096, True), (6144, False)])
+def test_panel_every_workgroup_full(n, f64):
+    bfa = _load()
+    rng = np.random.default_rng(n)
+    M = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))).astype(np.complex128 if f64 else np.complex64)
+    A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+    info, piv = _factor(bfa, A, f64)
+    assert info == 0
+    _check_factors(M, A, piv, f64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f64", [True, False])
+@pytest.mark.parametrize("n,lda", [(300, 301), (513, 1000)])
+def test_panel_leading_dimension(n, lda, f64):
+    """Columns further apart than their length: nothing between them is touched."""
+    bfa = _load()
+    rng = np.random.default_rng(lda)
+    M = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))).astype(np.complex128 if f64 else np.complex64)
+    A = torch.full((n, lda), 7 - 3j, dtype=torch.complex128 if f64 else torch.complex64, device="cuda")
+    A[:, :n] = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+    piv = torch.zeros(n, dtype=torch.int32, device="cuda")
+    assert (bfa.lu_factor if f64 else bfa.lu_factor_c)(A, n, piv, lda=lda) == 0
+    _check_factors(M, A[:, :n], piv.cpu().numpy(), f64)
+    assert (A[:, n:] == 7 - 3j).all()
+
+
+@pytest.mark.gpu
+def test_panel_sequence_numbers_restart():
+    """The exchange's 24-bit sequence numbers run out within a factorisation:
+    they begin again at 1, and words of the first use of these numbers are gone."""
+    import ctypes
+    bfa = _load()
+    lib = bfa.lib()
+    lib.bfa_xpanel_seq.restype = ctypes.c_uint
+    for k, n in enumerate((600, 520, 700, 600)):
+        rng = np.random.default_rng(k)
+        M = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+        A = torch.from_numpy(np.ascontiguousarray(M.T)).cuda()
+        if k == 1:
+            lib.bfa_xpanel_seq((1 << 24) - 300)
+        info, piv = _factor(bfa, A, True)
+        assert info == 0
+        _check_factors(M, A, piv, True)
+        if k == 1:
+            assert 1 < lib.bfa_xpanel_seq(0) < 1000
