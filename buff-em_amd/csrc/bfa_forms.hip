@@ -56,8 +56,22 @@ __global__ void k_c2z_add(const c2 *D, int64_t ldd, z2 *X, int64_t ldx, int m, i
 // for the chunk staged in LDS.
 #define RES_CHUNK 256
 #define RES_MAXRHS 8
-// right-hand sides of one launch: bounds the partials at what a batch needs
+// most right-hand sides of one launch
 #define RES_BATCH 32
+
+// Right-hand sides of one launch: groups of RES_MAXRHS side by side until the
+// launch has about 2,048 workgroups.  The partials grow with them (at
+// n = 20,000, 0.2 GB a group), so a matrix that fills the chip by itself takes
+// its groups one after the other, in no more memory than one needs.  With 32
+// right-hand sides, one group at a time against four: 1.02 -> 0.78 ms at
+// n = 1,350, 4.21 -> 3.74 at 5,760, 10.6 -> 10.5 at 11,400, 28.0 -> 27.9 at
+// 19,872 (whole call).
+static int residual_batch(int n, int nrhs)
+{
+  const int64_t nblk = (n + 255) / 256, wgs = nblk * ((n + RES_CHUNK - 1) / RES_CHUNK);
+  const int groups = (int)std::min<int64_t>(RES_BATCH / RES_MAXRHS, std::max<int64_t>(1, (2048 + wgs - 1) / wgs));
+  return std::min(nrhs, groups * RES_MAXRHS);
+}
 
 // Columns of a chunk.  A thread walks its chunk serially, so what bounds a
 // small system is the length of the chunk and the number of workgroups: at
@@ -172,6 +186,14 @@ extern "C" int bfa_lu_solve_c(const void *d_A, int n, int64_t lda, const int *d_
 
 // Mixed-precision solve with FP64 iterative refinement.  d_B (n x nrhs,
 // complex128) holds the right-hand sides on entry and the solution on exit.
+// bytes of the residual's partials in bfa_solve_refine's workspace
+extern "C" size_t bfa_refine_partials(int n, int nrhs)
+{
+  const int nres = residual_batch(n, nrhs);
+  const int chunk = residual_chunk((n + 255) / 256, n, (nres + RES_MAXRHS - 1) / RES_MAXRHS);
+  return (size_t)((n + chunk - 1) / chunk) * nres * n * sizeof(z2);
+}
+
 extern "C" int bfa_solve_refine(const void *d_M64, int64_t ldm, const void *d_LU32, int64_t ldlu, const int *d_ipiv,
                                 int n, void *d_B, int nrhs, int64_t ldb, double tol, int maxit, int *iters,
                                 double *resid, void *stream)
@@ -180,12 +202,12 @@ extern "C" int bfa_solve_refine(const void *d_M64, int64_t ldm, const void *d_LU
     return fail(BFA_ERR_ARG, "bfa_solve_refine: bad argument");
   hipStream_t st = (hipStream_t)stream;
   if (maxit <= 0) maxit = 10;
-  const int nblk = (n + 255) / 256, nres = std::min(nrhs, RES_BATCH);
+  const int nblk = (n + 255) / 256, nres = residual_batch(n, nrhs);
   const int chunk = residual_chunk(nblk, n, (nres + RES_MAXRHS - 1) / RES_MAXRHS);
   const int nchunk = (n + chunk - 1) / chunk;
   const size_t zsz = (size_t)n * nrhs * sizeof(z2);
   // workspace: B copy (z), X (z), R (z), D (c), partials, norms, solve scratch
-  const size_t part = (size_t)nchunk * nres * n * sizeof(z2);
+  const size_t part = bfa_refine_partials(n, nrhs);
   const size_t norms_b = (size_t)2 * nblk * nrhs * sizeof(double);
   const size_t scr = bfa::lu_solve_scratch_bytes(n, nrhs, 8);
   char *w = nullptr;
@@ -215,9 +237,9 @@ extern "C" int bfa_solve_refine(const void *d_M64, int64_t ldm, const void *d_LU
   rc = bfa::lu_solve_prep_c(d_LU32, n, ldlu, d_ipiv, st, scratch);
   for (it = 0; rc == BFA_OK && it <= maxit; it++) {
     if (it > 0) {
-      // r = b - M64 x, RES_BATCH right-hand sides at a time
-      for (int j0 = 0; j0 < nrhs; j0 += RES_BATCH) {
-        const int nj = std::min(RES_BATCH, nrhs - j0);
+      // r = b - M64 x, nres right-hand sides at a time
+      for (int j0 = 0; j0 < nrhs; j0 += nres) {
+        const int nj = std::min(nres, nrhs - j0);
         hipLaunchKernelGGL(k_residual_part, dim3(nblk, nchunk, (nj + RES_MAXRHS - 1) / RES_MAXRHS), dim3(256), 0, st,
                            M, ldm, n, (const z2 *)(X + (size_t)j0 * n), (int64_t)n, nj, chunk, P);
         hipLaunchKernelGGL(k_residual_final, dim3(nblk, nj), dim3(256), 0, st, (const z2 *)P, nchunk, n, nj,
