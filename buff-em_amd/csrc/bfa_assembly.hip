@@ -1303,7 +1303,10 @@ __device__ __forceinline__ void far_gather_tile(const DevGeom &g, double kre, do
 }
 
 // NC: most distinct tetrahedra of a tile (31 on average on the Kuhn spheres,
-// 34 at most; 64 is any mesh's bound)
+// 34 at most; 64 is any mesh's bound).  64 slots hold 49 KB of LDS, three
+// workgroups a CU, 40 hold 35 KB, four: N = 19,872 assembled in 8.5 ms with the
+// tetrahedra in the mesh's order and 12.5 in random order, which needs the 64
+// and gathers records further apart (all moments in LDS: 17.0 and 27.2)
 template <int NC>
 __global__ __launch_bounds__(GS_NT, 4) void k_far_gather(DevGeom g, double kre, double kim,
                                                       const double *__restrict__ tpt, cd *M, int64_t ld, int ntiles)

@@ -1271,7 +1271,7 @@ static int tail_rows(bool f64, hipStream_t st, const LUWork *lw)
 }
 
 // Columns [j0, n) of a matrix whose remaining rows fit the register panel, on
-// one stream: a 256-column panel costs ~2 us a column whatever its height,
+// one stream: a 256-column panel costs 1.5 to 2.9 us a column by its height,
 // against ~5 us a column plus seven TRSM / GEMM / swap launches per 256
 // columns in the recursive panel, and the update of so small a remainder is
 // shorter than what overlapping it with the next panel would save.

@@ -139,7 +139,10 @@ int  bfa_fibbi_preload(bfa_geometry *g, const char *path, int td_order, int64_t 
 
 /* ---- warm step: VIE matrix --------------------------------------------- */
 /* SWGGeometry::AssembleVIEMatrix (VIEMatrix.cc:431-460): d_M (N x N,
- * complex128, ld >= N) receives G + chi^-1 block, both triangles.        */
+ * complex128, ld >= N) receives G + chi^-1 block, both triangles.
+ * Assemblies of one geometry share its work space: calls on several streams
+ * or threads take turns on the device; replays of captured calls are ordered
+ * by the caller.                                                          */
 int  bfa_assemble_vie(bfa_geometry *g, double omega_re, double omega_im,
                       const bfa_material *mat, void *d_M, int64_t ld, void *stream);
 
