@@ -863,6 +863,15 @@ __device__ __forceinline__ unsigned long long panel_key(float v, int row)
   return ((unsigned long long)__float_as_uint(v) << 32) | (unsigned long long)(0xFFFFFFFFu - (unsigned)row);
 }
 
+// A row's magnitude in the search.  NaN, which compares with nothing, ranks as
+// zero: a column of NaN would have no candidate, and "no row" taken as a pivot
+// would send the interchanges to row -1.
+template <typename T> __device__ __forceinline__ T pivot_mag(cplx<T> x)
+{
+  const T v = c_abs1(x);
+  return v == v ? v : (T)0;
+}
+
 // Body shared by the single-matrix and the grouped panel kernels: workgroup
 // g of the nwg that factor this panel; rows = the workgroup's LDS block.
 // Per column: the workgroup's candidate (found while updating the previous
@@ -894,7 +903,7 @@ __device__ __forceinline__ void panel_body(cplx<T> *A, int m, int w, int64_t lda
   int brow = INT_MAX;
   for (int r = tid; r < nr; r += blockDim.x) {
     int dummy = 0;
-    argmax_merge(best, brow, dummy, c_abs1(RW(r, 0)), r0 + r, 0);
+    argmax_merge(best, brow, dummy, pivot_mag(RW(r, 0)), r0 + r, 0);
   }
   for (int j = 0; j < w; j++) {
     const int buf = j & 1;
@@ -927,7 +936,8 @@ __device__ __forceinline__ void panel_body(cplx<T> *A, int m, int w, int64_t lda
       if (tid == 0) sh.wrow[0] = (int)(0xFFFFFFFFu - (unsigned)k);
     }
     __syncthreads();
-    const int p = sh.wrow[0], win = p / rpw;
+    // (a row of the panel also where a barrier gave up and no key came)
+    const int p = max(j, min(m - 1, sh.wrow[0])), win = p / rpw;
     if (tid < PW) {
       const cplx<T> *d = &rdata[((size_t)buf * nwg + win) * PW + tid];
       sh.prow[tid] = tid < w ? cplx<T>{ld_agent(&d->re), ld_agent(&d->im)} : cplx<T>{0, 0};
@@ -962,7 +972,7 @@ __device__ __forceinline__ void panel_body(cplx<T> *A, int m, int w, int64_t lda
       }
       if (j + 1 < w) {
         int dummy = 0;
-        argmax_merge(best, brow, dummy, c_abs1(RW(r, j + 1)), gr, 0);
+        argmax_merge(best, brow, dummy, pivot_mag(RW(r, j + 1)), gr, 0);
       }
     }
   }

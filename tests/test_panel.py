@@ -157,6 +157,14 @@ def test_panel_workgroups_run_at_once(f64):
                 assert rows == (fits[0] if fits else 0)
 
 
+def _masked_stream(hip):
+    import ctypes
+    h = ctypes.c_void_p()
+    mask = (ctypes.c_uint32 * 8)(0xFFFFFFFF)
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(h), 8, mask) == 0
+    return h, torch.cuda.ExternalStream(h.value)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("f64", [True, False])
 def test_panel_on_a_stream_with_part_of_the_cus(f64):
@@ -165,10 +173,7 @@ def test_panel_on_a_stream_with_part_of_the_cus(f64):
     bfa = _load()
     torch.zeros(1, device="cuda")
     hip = ctypes.CDLL("libamdhip64.so")
-    mask = (ctypes.c_uint32 * 8)(0xFFFFFFFF)
-    h = ctypes.c_void_p()
-    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(h), 8, mask) == 0
-    st = torch.cuda.ExternalStream(h.value)
+    h, st = _masked_stream(hip)
     n = 1350
     rng = np.random.default_rng(2)
     M = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))).astype(np.complex128 if f64 else np.complex64)
@@ -247,3 +252,43 @@ def test_panel_sequence_numbers_restart():
         _check_factors(M, A, piv, True)
         if k == 1:
             assert 1 < lib.bfa_xpanel_seq(0) < 1000
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["nan", "inf", "column", "underflow"])
+@pytest.mark.parametrize("path", ["registers", "lds", "tall", "local"])
+def test_lu_of_values_that_are_not_numbers(path, kind):
+    """NaN in a matrix (a permittivity of exactly 1 puts it there), infinities,
+    and entries whose squares underflow in complex64: every panel still chooses
+    rows of its own, the factors carry the NaN on, and the solve ends."""
+    import ctypes
+    bfa = _load()
+    n = 6400 if path == "tall" else 300
+    g = torch.Generator(device="cuda").manual_seed(n)
+    M = torch.complex(*[torch.randn(n, n, generator=g, device="cuda") for _ in range(2)])
+    if kind == "nan":
+        M.fill_(complex("nan"))
+    elif kind == "inf":
+        M[3, 5] = float("inf")
+    elif kind == "column":
+        M[17] = complex("nan")
+    else:
+        M *= 1e-30
+    piv = torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    factor = bfa.lu_factor_c_local if path == "local" else bfa.lu_factor_c
+    if path == "lds":
+        hip = ctypes.CDLL("libamdhip64.so")
+        h, st = _masked_stream(hip)
+        factor(M, n, piv, stream=st)
+        torch.cuda.synchronize()
+        assert hip.hipStreamDestroy(h) == 0
+    else:
+        factor(M, n, piv)
+    p = piv.cpu().numpy()
+    assert ((p >= np.arange(n)) & (p < n)).all()
+    assert not bool(torch.isfinite(torch.view_as_real(M)).all())
+    B = torch.ones((2, n), dtype=torch.complex64, device="cuda")
+    bfa.lu_solve_c(M, n, piv, B, 2)
+    torch.cuda.synchronize()
+    assert not bool(torch.isfinite(torch.view_as_real(B)).all())
