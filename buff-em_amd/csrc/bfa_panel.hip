@@ -19,12 +19,15 @@ template <typename T> struct zc { T re, im; };
 template <typename T> __device__ __forceinline__ zc<T> z_mul(zc<T> a, zc<T> b)
 { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 template <typename T> __device__ __forceinline__ T t_fma(T a, T b, T c) { return sizeof(T) == 8 ? (T)fma(a, b, c) : (T)fmaf(a, b, c); }
-// a - l u
+// l u, apart from the sum it goes into, so that one rounding and not two is at
+// the sum's magnitude (random matrices: factor error 10 % less, 1 % of the time)
+template <typename T> __device__ __forceinline__ zc<T> z_prod(zc<T> l, zc<T> u)
+{ return {t_fma(-l.im, u.im, l.re * u.re), t_fma(l.im, u.re, l.re * u.im)}; }
+// a - l u, a + l u
 template <typename T> __device__ __forceinline__ zc<T> z_fms(zc<T> a, zc<T> l, zc<T> u)
-{ return {t_fma(l.im, u.im, t_fma(-l.re, u.re, a.re)), t_fma(-l.im, u.re, t_fma(-l.re, u.im, a.im))}; }
-// a + l u
+{ const zc<T> p = z_prod(l, u); return {a.re - p.re, a.im - p.im}; }
 template <typename T> __device__ __forceinline__ zc<T> z_fma(zc<T> a, zc<T> l, zc<T> u)
-{ return {t_fma(-l.im, u.im, t_fma(l.re, u.re, a.re)), t_fma(l.im, u.re, t_fma(l.re, u.im, a.im))}; }
+{ const zc<T> p = z_prod(l, u); return {a.re + p.re, a.im + p.im}; }
 template <typename T> __device__ __forceinline__ zc<T> z_sub(zc<T> a, zc<T> b) { return {a.re - b.re, a.im - b.im}; }
 template <typename T> __device__ __forceinline__ zc<T> z_pick(bool c, zc<T> a, zc<T> b)
 { return {c ? a.re : b.re, c ? a.im : b.im}; }
@@ -175,11 +178,13 @@ template <typename T, int R, int AL> struct XpShared {
 // at its own magnitude about 10 times a panel and not once a column, as with
 // the panels of 32 columns and the GEMM that accumulates from zero.
 // |PA - LU| / |A| over u, complex64, VIE matrices of 270, 1,350 and 3,822
-// unknowns: 0.82, 1.22, 1.58; subtracted from the entries product by product
-// 4.8, 7.5, 9.3, by 32-column panels 1.55, 1.87, 2.20.  On random matrices all
-// agree to 5 %; sums over the whole panel are 3 % worse there and better on
-// the VIE matrices (0.66, 1.00, 1.44).  No slower: the values, read by row
-// index, need no branch tree, and a column's time is the exchange's.
+// unknowns: 0.82, 1.20, 1.57; subtracted from the entries product by product
+// 4.8, 7.5, 9.3, by 32-column panels 1.55, 1.87, 2.20.  Random matrices of 200
+// and 512, complex128: 15.5 and 36.9, 32-column panels 16.4 and 39.9.  Sums
+// over the whole panel are better on the VIE matrices (0.66, 1.00, 1.44) and
+// 4 % worse on random ones.  About as fast (n = 1,350 3.49 -> 3.57 ms): the
+// values, read by row index, need no branch tree, and a column's time is the
+// exchange's.
 // Lanes also hold, redundantly in every wave, the next two columns row by row
 // (lane = row), so that the multipliers of column j, the values of column
 // j + 1 and its pivot candidate need no workgroup reduction.
