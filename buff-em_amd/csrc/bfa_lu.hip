@@ -1281,11 +1281,11 @@ static int tail_rows(bool f64, hipStream_t st, const LUWork *lw)
 }
 
 // Columns [j0, n) of a matrix whose remaining rows fit the register panel, on
-// one stream: a 256-column panel costs 1.5 to 2.9 us a column by its height,
+// one stream: a 256-column panel costs 1.5 to 3.0 us a column by its height,
 // against ~5 us a column plus seven TRSM / GEMM / swap launches per 256
 // columns in the recursive panel, and the update of so small a remainder is
 // shorter than what overlapping it with the next panel would save.
-// Factorisation, complex128: 2.07 -> 0.7 ms at n = 270, 9.8 -> 3.6 ms at
+// Factorisation, complex128: 2.07 -> 0.67 ms at n = 270, 9.8 -> 3.57 ms at
 // n = 1,350.
 template <typename T>
 static int lu_factor_tail(cplx<T> *A, int n, int64_t lda, int *ipiv, hipStream_t st, int j0, LUWork *lw)

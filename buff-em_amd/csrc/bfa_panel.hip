@@ -494,10 +494,10 @@ void xpanel_carve(bool f64, char *mem, XPanel *p)
 // Rows a workgroup holds, fewest first: a column's time grows with them (the
 // register update outlasts the exchange from about 16 complex128 / 32
 // complex64 rows), the exchange's hardly with the workgroups.  Measured, us a
-// column of 256: complex128 1.74 (8 rows, m = 256), 2.10 (16, 1,350), 2.69
-// (24, 3,000), 2.87 (32, 4,000); complex64 1.46 (8, 256), 1.75 (16, 1,350),
-// 2.30 (32, 4,000), 2.71 (48, 6,000); with an interchange in every column 2.18
-// to 3.85 and 1.74 to 3.36.
+// column of 256: complex128 1.76 (8 rows, m = 256), 2.18 (16, 1,350), 2.75
+// (24, 3,000), 3.03 (32, 4,000); complex64 1.48 (8, 256), 1.78 (16, 1,350),
+// 2.36 (32, 4,000), 2.85 (48, 6,000); with an interchange in every column 2.21
+// to 3.97 and 1.75 to 3.48.
 // A panel's workgroups wait for each other, so all must run at once: XP_MAXWG
 // of them at most, and what the device holds (a partition of it has fewer CUs).
 int xpanel_max_rows(bool f64)
